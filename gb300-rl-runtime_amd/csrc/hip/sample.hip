@@ -5,8 +5,9 @@
 // HBM-streaming kernels. Batches with top-k take one workgroup per row that
 // streams the row in chunks (sample_stream_kernel, below) when the rows are at
 // most 32,768 logits or number at least kStreamMinRows, and split + merge when
-// fewer long rows would leave most compute units idle. Vocabularies above
-// 32,768 without top-k (or greedy) take split + merge too; the others
+// fewer long rows would leave most compute units idle. Greedy batches of
+// vocabularies above 32,768 take split + merge too, batches without top-k of
+// such vocabularies the passes of sample_nucleus.h over the slices; the others
 // (whole-vocabulary nucleus, greedy) one workgroup per row holding the row in
 // registers (sample_row_kernel, below).
 //
@@ -36,9 +37,9 @@
 //         chosen bin holds at most 64 keys; rank sort of the kept set by
 //         (x desc, index asc); 24-bit integer weights rl_sample_weight(x -
 //         max), nucleus prefix and the ascending-index integer CDF walk - in
-//         one wave when at most 64 elements are kept. Rows without top-k (a
-//         whole-vocabulary nucleus) or whose candidates overflow take the
-//         exact full-row path below.
+//         one wave when at most 64 elements are kept. Rows without top-k (in
+//         a batch with per-row top-k) or whose candidates overflow take the
+//         exact full-row path.
 // Integer weights make every sum exact, so the token is bit-identical to the
 // host restatement whatever the reduction order.
 #include <hip/hip_runtime.h>
@@ -50,6 +51,7 @@
 #include "rl_sample_math.h"
 #include "sample.h"
 #include "sample_core.h"
+#include "sample_nucleus.h"
 
 namespace {
 
@@ -838,8 +840,9 @@ extern "C" int rl_hip_sample(const rl_sample_args_t *a)
     // Rows without top-k whose whole row fits one workgroup's registers: the
     // row kernel. Batches with top-k: the stream kernel when the rows are
     // short or fill most of the device (one row per compute unit, so fewer
-    // long rows leave it idle), else split and merge. Everything else: split
-    // and merge.
+    // long rows leave it idle), else split and merge. Long rows without
+    // top-k: the slice passes of sample_nucleus.h (faster than split + merge
+    // at 1 to 512 rows, measured there). Long greedy rows: split and merge.
     const bool no_topk = !a->top_k && (a->top_k_all == 0 || a->top_k_all >= a->vocab);
     if (a->vocab <= kRowVocab && (no_topk || a->greedy)) {
         hipLaunchKernelGGL(sample_row_kernel, dim3(a->rows), dim3(kMergeThreads), 0, rl_stream(), p);
@@ -848,6 +851,23 @@ extern "C" int rl_hip_sample(const rl_sample_args_t *a)
     if (!no_topk && !a->greedy && (a->vocab <= kRowVocab || a->rows >= kStreamMinRows)) {
         hipLaunchKernelGGL(sample_stream_kernel, dim3(a->rows), dim3(kMergeThreads), 0, rl_stream(), p);
         return rl_check_launch("sample_stream_kernel launch");
+    }
+    if (no_topk && !a->greedy) {
+        // (one workgroup per slice, a row's slices on one XCD: nuc_place)
+        const dim3 grid((a->rows + kNucXcds - 1) / kNucXcds * kNucXcds * p.splits);
+        hipLaunchKernelGGL(nucleus_split_kernel, grid, dim3(kThreads), 0, rl_stream(), p);
+        if (rl_check_launch("nucleus_split_kernel launch"))
+            return -1;
+        hipLaunchKernelGGL(nucleus_weigh_kernel, grid, dim3(kMergeThreads), 0, rl_stream(), p);
+        if (rl_check_launch("nucleus_weigh_kernel launch"))
+            return -1;
+        if (a->top_p || (a->top_p_all > 0.f && a->top_p_all < 1.f)) {
+            hipLaunchKernelGGL(nucleus_edge_kernel, grid, dim3(kMergeThreads), 0, rl_stream(), p);
+            if (rl_check_launch("nucleus_edge_kernel launch"))
+                return -1;
+        }
+        hipLaunchKernelGGL(nucleus_pick_kernel, dim3(a->rows), dim3(kMergeThreads), 0, rl_stream(), p);
+        return rl_check_launch("nucleus_pick_kernel launch");
     }
     hipLaunchKernelGGL(sample_split_kernel, dim3(p.splits, a->rows),
                        dim3(kThreads), 0, rl_stream(), p);

@@ -235,3 +235,54 @@ def test_greedy_long_rows_repeated_calls(rl, gpu, orc, olib):
         print(f"[sample] greedy call {it}: {rows} x {vocab}", flush=True)
         tok = _check(rl, orc, olib, x, vocab=vocab, greedy=True)
         assert tok[0] == np.flatnonzero(x[0, :vocab] == np.float32(6.0)).min()
+
+
+@pytest.mark.parametrize("rows,vocab,stride", [(1, 32769, 32772), (9, 65536, 65536), (17, 40961, 40964),
+                                               (3, 524288, 524288)])
+def test_sliced_nucleus_edges(rl, gpu, orc, olib, rows, vocab, stride):
+    """Rows without top-k above the row kernel's size, over the slices: one
+    slice past a boundary, rows that leave XCDs without a row, the most slices
+    (64); dense and sparse boundaries, massive ties in the boundary bin (its
+    lists overflow: the exact path), -inf rows, top-p 1."""
+    rng = np.random.default_rng(vocab + rows)
+    x = np.full((rows, stride), np.float32(9.0))             # padding past vocab never read
+    x[:, :vocab] = rng.standard_normal((rows, vocab), dtype=np.float32)
+    if rows > 2:
+        x[1, :vocab] = np.round(x[1, :vocab])                # ties: more members than a slice lists
+        x[2, :vocab] = -np.inf
+    if rows > 8:
+        x[3, :vocab] = 0.25                                  # every logit equal
+        x[4, : vocab - 1] = -np.inf
+        x[5, :vocab] = np.sort(x[5, :vocab])                 # one slice holds the whole boundary bin
+        x[6, :vocab] -= 18.0
+        x[6, 77] = 0.0                                       # the rest weighs next to nothing
+    seeds = rng.integers(0, 2**63, rows, dtype=np.uint64)
+    for p in (0.05, 0.9, 0.999, 1.0):
+        _check(rl, orc, olib, x, vocab=vocab, temperature=0.9, top_k=0, top_p=p, seeds=seeds, step=int(p * 1000))
+
+
+def test_sliced_nucleus_per_row_parameters(rl, gpu, orc, olib):
+    """Per-row temperature and top-p over 40,000 logits with no top-k: greedy
+    rows (temperature 0), nucleus rows and rows with top-p 1 in one call."""
+    rows, V = 21, 40000
+    rng = np.random.default_rng(4243)
+    x = rng.standard_normal((rows, V), dtype=np.float32)
+    temp = rng.choice(np.float32([0.0, 0.6, 1.0, 1.7]), rows).astype(np.float32)
+    topp = rng.choice(np.float32([1.0, 0.95, 0.3]), rows).astype(np.float32)
+    bufs = [rl.DeviceBuffer.from_array(a) for a in (x, temp, topp)]
+    tok, lp = rl.DeviceBuffer(rows * 4), rl.DeviceBuffer(rows * 4)
+    a = rl.sample_args(bufs[0], rows, V, V, tok, lp, seed=5, step=7)
+    a.temperature, a.top_p = bufs[1].ptr, bufs[2].ptr
+    ws = rl.sample_workspace(a)
+    rl.sample(a)
+    rl.sync()
+    gt, gl = tok.download(np.uint32, rows), lp.download(np.float32, rows)
+    import ctypes as C
+    lpv = C.c_double()
+    for r in range(rows):
+        want = olib.orc_sample_row(x[r].ctypes.data, V, int(not temp[r] > 0), float(temp[r]), 0, float(topp[r]), 5, 7,
+                                   r, C.byref(lpv))
+        assert gt[r] == want, (r, temp[r], topp[r], gt[r], want)
+        assert abs(gl[r] - lpv.value) < 1e-4, r
+    for b in bufs + [tok, lp, ws]:
+        b.close()
