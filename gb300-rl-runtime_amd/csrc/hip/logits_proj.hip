@@ -8,6 +8,8 @@
 //
 //  tiles   one 512-thread workgroup (8 waves, 4 along M x 2 along N) per
 //          output tile, K in steps of 64:
+//          - up to 128 rows: tiles of 32, 64 or 128 rows by 64 or 128
+//            (logits_proj_rows_kernel, below).
 //          - up to 256 rows: 256 x 128 tiles, waves of 64 x 64 (4 x 4 MFMA
 //            blocks of 16 x 16), a 3-stage LDS ring (144 KiB). Every W tile
 //            is read by exactly one workgroup, and the grid (one workgroup
@@ -201,6 +203,134 @@ __global__ __launch_bounds__(kThreads) void logits_proj_kernel(ProjParams p)
         }
 }
 
+// ---- up to 128 rows: the W stream ----------------------------------------------
+// Bound: the HBM stream of W (262 MB at 32,000 x 4,096: 43 us at the 6 TB/s a
+// read stream reaches here). The 256-row tile spends two thirds of its copies
+// on X rows that are not there, and its one 144 KiB workgroup per compute unit
+// keeps 32 KiB of W in flight. Here every workgroup covers all rows of X, so W
+// is read once, and the tiles are small: WN waves of TNR x 16 vocabulary rows
+// each, a 3-stage ring of 12 to 32 KiB stages, so that up to four workgroups
+// share a compute unit and fill each other's barrier waits. (Deeper rings with
+// fewer workgroups were slower: 6 stages 52 us against 45 at 24 rows.)
+// Each workgroup starts at another K step and wraps, so that the workgroups
+// that run at once read W at different columns; all starting at 0 they read
+// column k of rows 8 KiB apart together (24 rows 51.8 us against 45.5).
+// Measured back to back over three copies of W, 32,000 x 4,096 (us, against
+// the 256 x 128 tile): 1 row 44.4 (60.4), 24 rows 45.5 (62.9), 64 rows 48.8
+// (65.4), 128 rows 55.9 (70.5); 20 rows of 17,393 x 2,048 12.3 (30); 1 row of
+// 8,001 x 1,024 5.6 (15.0). W straight to registers (no LDS; every wave reads
+// X from L2) took 57 to 111 us at 24 rows.
+template <int TMR, int TNR, int WN>
+struct RowsTile {
+    static constexpr int NSTAGE = 3;
+    static constexpr int M = TMR * 16;
+    static constexpr int N = WN * TNR * 16;
+    static constexpr int XBYTES = M * BK * 2;
+    static constexpr int WBYTES = N * BK * 2;
+    static constexpr int STAGE = XBYTES + WBYTES;
+    static constexpr int XOPS = XBYTES / 1024 / WN;  // 1 KiB copies per wave and step
+    static constexpr int WOPS = WBYTES / 1024 / WN;
+    static_assert(XOPS * 1024 * WN == XBYTES && WOPS * 1024 * WN == WBYTES, "whole copies per wave");
+};
+
+template <int TMR, int TNR, int WN>
+__global__ __launch_bounds__(WN * 64) void logits_proj_rows_kernel(ProjParams p)
+{
+    using T = RowsTile<TMR, TNR, WN>;
+    constexpr int NS = T::NSTAGE;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[NS * T::STAGE];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t n0 = blockIdx.x * T::N;
+    const int fr = lane & 15, fc = lane >> 4;
+
+    rl_f32x4 acc[TMR][TNR];
+#pragma unroll
+    for (int i = 0; i < TMR; i++)
+#pragma unroll
+        for (int j = 0; j < TNR; j++)
+            acc[i][j] = rl_f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const uint32_t ksteps = p.K / BK;
+    uint32_t xoff[T::XOPS], woff[T::WOPS];
+    piece_offsets<T::XOPS>(p.ldx, p.M, 0, wave * T::XOPS, lane, xoff);
+    piece_offsets<T::WOPS>(p.ldw, p.N, n0, wave * T::WOPS, lane, woff);
+    const uint16_t *wbase = p.w + (size_t)n0 * p.ldw;
+    const uint32_t rot = blockIdx.x / kXcds * 5u % ksteps;
+    auto stage = [&](uint32_t kt) {
+        RL_LDS uint8_t *b = (RL_LDS uint8_t *)(smem + (kt % NS) * T::STAGE);
+        const uint32_t k = kt + rot < ksteps ? kt + rot : kt + rot - ksteps;
+        stage_rows<T::XOPS>(p.x + k * BK, xoff, b, wave * T::XOPS);
+        stage_rows<T::WOPS>(wbase + k * BK, woff, b + T::XBYTES, wave * T::WOPS);
+    };
+#pragma unroll
+    for (int s = 0; s < NS - 1; s++)
+        if ((uint32_t)s < ksteps)
+            stage(s);
+    for (uint32_t kt = 0; kt < ksteps; kt++) {
+        // as in logits_proj_kernel: this wave's copies of step kt have landed
+        // once only those of step kt + 1 are outstanding; after the barrier
+        // every wave's have, and the buffer of step kt - 1 is free
+        if (kt + 1 < ksteps)
+            rl_wait_vmcnt<T::XOPS + T::WOPS>();
+        else
+            rl_wait_vmcnt<0>();
+        __syncthreads();
+        if (kt + NS - 1 < ksteps)
+            stage(kt + NS - 1);
+        RL_LDS const uint8_t *xs = (RL_LDS const uint8_t *)(smem + (kt % NS) * T::STAGE);
+        RL_LDS const uint8_t *ws = xs + T::XBYTES;
+#pragma unroll
+        for (int s = 0; s < BK / 32; s++) {
+            s16x8 af[TMR], bf[TNR];
+            const int c = 4 * s + fc;
+#pragma unroll
+            for (int i = 0; i < TMR; i++) {
+                const int ra = i * 16 + fr;
+                af[i] = *(RL_LDS const s16x8 *)(xs + ra * (BK * 2) + ((c ^ (ra & 7)) << 4));
+            }
+#pragma unroll
+            for (int j = 0; j < TNR; j++) {
+                const int rb = (wave * TNR + j) * 16 + fr;
+                bf[j] = *(RL_LDS const s16x8 *)(ws + rb * (BK * 2) + ((c ^ (rb & 7)) << 4));
+            }
+#pragma unroll
+            for (int i = 0; i < TMR; i++)
+#pragma unroll
+                for (int j = 0; j < TNR; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[i]),
+                                                                        __builtin_bit_cast(bf16x8, bf[j]),
+                                                                        acc[i][j], 0, 0, 0);
+        }
+    }
+
+#pragma unroll
+    for (int i = 0; i < TMR; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uint32_t m = i * 16 + 4 * fc + r;
+            if (m >= p.M)
+                continue;
+            float *orow = p.out + (size_t)m * p.ldo;
+#pragma unroll
+            for (int j = 0; j < TNR; j++) {
+                const uint32_t n = n0 + (wave * TNR + j) * 16 + fr;
+                if (n < p.N)
+                    orow[n] = acc[i][j][r];
+            }
+        }
+}
+
+template <int TMR, int TNR, int WN>
+int launch_rows(const ProjParams &p)
+{
+    constexpr uint32_t per = RowsTile<TMR, TNR, WN>::N;
+    const uint64_t grid = ((uint64_t)p.N + per - 1) / per;
+    hipLaunchKernelGGL((logits_proj_rows_kernel<TMR, TNR, WN>), dim3((uint32_t)grid), dim3(WN * 64), 0,
+                       rl_stream(), p);
+    return rl_check_launch("logits_proj_rows_kernel launch");
+}
+
 template <int TN>
 int launch_proj(ProjParams p)
 {
@@ -246,6 +376,15 @@ extern "C" int rl_hip_logits_proj(const rl_logits_proj_args_t *a)
     p.ldx = a->x_stride;
     p.ldw = a->w_stride;
     p.ldo = a->logits_stride;
+    // up to 128 rows the W stream (tiles of just enough rows; measured at the
+    // kernel); above, where the matrix cores weigh as much as the stream, the
+    // large tiles:
+    if (a->rows <= 32)
+        return launch_rows<2, 1, 4>(p);
+    if (a->rows <= 64)
+        return launch_rows<4, 1, 8>(p);
+    if (a->rows <= 128)
+        return launch_rows<8, 2, 4>(p);
     // above 256 rows the 256 x 256 tile (more MFMA work per LDS byte); up to
     // 256 rows the 256 x 128 tile, whose grid still fills the device
     return a->rows > (uint32_t)BM ? launch_proj<8>(p) : launch_proj<4>(p);

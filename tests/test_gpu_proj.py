@@ -45,12 +45,20 @@ def _case(rl, rows, vocab, hidden, seed, check_rows=None, check_cols=None, repea
         b.close()
 
 
-# up to 256 rows the 256 x 128 tile, above it the 256 x 256 tile (three M
+# 129 to 256 rows the 256 x 128 tile, above it the 256 x 256 tile (three M
 # tiles and a partial N tile at 700 x 777)
 @pytest.mark.parametrize("rows,vocab,hidden", [(1, 129, 64), (130, 1000, 128), (64, 32000, 256),
                                                (256, 130, 192), (200, 4000, 128), (257, 300, 4096),
                                                (700, 777, 192)])
 def test_projection_shapes(rl, gpu, rows, vocab, hidden):
+    _case(rl, rows, vocab, hidden, seed=rows + vocab + hidden)
+
+
+# the tiles of up to 128 rows, at their row limits; vocabularies that end inside
+# a tile and a 16-column block; one, two and more K steps than pipeline stages
+@pytest.mark.parametrize("rows", [1, 17, 32, 33, 64, 65, 128, 129])
+@pytest.mark.parametrize("vocab,hidden", [(1, 64), (63, 128), (191, 192), (1025, 320)])
+def test_projection_few_rows(rl, gpu, rows, vocab, hidden):
     _case(rl, rows, vocab, hidden, seed=rows + vocab + hidden)
 
 
