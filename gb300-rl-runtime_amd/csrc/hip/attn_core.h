@@ -148,16 +148,25 @@ __device__ __forceinline__ uint32_t table_row_of(const AttnParams &p, uint32_t b
     return p.row_map ? rl_sload(p.row_map + b) : b;
 }
 struct CtxFromArray {
+    static constexpr bool kSettledWindow = false;
     const uint32_t *ctx;
     __device__ __forceinline__ uint32_t operator()(uint32_t b) const { return rl_sload(ctx + b); }
     __device__ __forceinline__ uint32_t table_row(const AttnParams &p, uint32_t b) const { return table_row_of(p, b); }
 };
 struct CtxFixed {
+    static constexpr bool kSettledWindow = false;
     uint32_t value;
     __device__ __forceinline__ uint32_t operator()(uint32_t) const { return value; }
     __device__ __forceinline__ uint32_t table_row(const AttnParams &p, uint32_t b) const { return table_row_of(p, b); }
 };
+// As CtxFixed, for a stream that is a chain of latencies and not of bytes (a
+// workgroup to itself): its table window is settled where it is loaded, see
+// Issuer::issue.
+struct CtxRow : CtxFixed {
+    static constexpr bool kSettledWindow = true;
+};
 struct CtxLds {
+    static constexpr bool kSettledWindow = false;
     RL_LDS const uint32_t *ctx;  // [batch]
     RL_LDS const uint32_t *row;  // [batch]: the table row of each rollout
     __device__ __forceinline__ uint32_t operator()(uint32_t b) const { return ctx[b]; }
@@ -192,6 +201,18 @@ struct Issuer {
         }
     }
 
+    // The compiler does not see the waits above, so it puts a vmcnt(0) of its
+    // own before every readlane of the window, which also waits for the tile
+    // in flight: one tile is copied while one is consumed. Where HBM is the
+    // bound that costs nothing (without it the fused step was slower, 127
+    // against 122 us); where latency is, redefining the window after its wait
+    // lets both stages' copies fly.
+    __device__ __forceinline__ void settle_window()
+    {
+        if constexpr (CtxFn::kSettledWindow)
+            asm volatile("" : "+v"(win0), "+v"(win1));
+    }
+
     __device__ __forceinline__ void set_rollout(const AttnParams &p, uint32_t nb)
     {
         b = nb;
@@ -215,6 +236,7 @@ struct Issuer {
             win0 = (lb + (uint32_t)lane < nblk) ? trow[lb + lane] : 0u;
             win1 = (lb + 64u + (uint32_t)lane < nblk) ? trow[lb + 64u + lane] : 0u;
             rl_wait_vmcnt<0>();
+            settle_window();
             wrow = row;
             wfirst = lb;
         }
@@ -311,6 +333,17 @@ __device__ __forceinline__ void row_begin(RowState<D, G, DT, TPB> &rs, RL_LDS co
     rs.bad = false;
 }
 
+// Max over the four lanes l % 16, l % 16 + 16, + 32, + 48 (every lane gets
+// it), by swapping halves and rows of 16: a few VALU cycles, where a shuffle
+// goes through the LDS crossbar.
+__device__ __forceinline__ float tile_max(float x)
+{
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // One staged tile: QK (MFMA), online softmax, PV (MFMA).
 template <int D, int G, int DT, int TPB, bool FULL>
 __device__ __forceinline__ void consume_tile(const AttnParams &p, RowState<D, G, DT, TPB> &rs,
@@ -341,8 +374,7 @@ __device__ __forceinline__ void consume_tile(const AttnParams &p, RowState<D, G,
         sv[r] = ok ? sc[r] * p.scale_log2 : -INFINITY;
     }
     float mx = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = tile_max(mx);
     const float m_new = fmaxf(rs.m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const bool grow = (m_new > rs.m_run) && (rs.m_run != -INFINITY);
@@ -351,7 +383,13 @@ __device__ __forceinline__ void consume_tile(const AttnParams &p, RowState<D, G,
         rs.l_run *= alpha;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const float a = __shfl(alpha, 4 * tg + r);
+            // head 4 tg + r's factor, from lane 4 tg + r; the rows past the
+            // group's heads hold zeros, whatever multiplies them
+            float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha), r));
+            if constexpr (G > 4) {
+                const float a4 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha), 4 + r));
+                a = tg == 0 ? a : a4;
+            }
 #pragma unroll
             for (int n = 0; n < C::NB; n++)
                 rs.acc[n][r] *= a;
@@ -491,6 +529,13 @@ __device__ __forceinline__ void wait_tiles(uint32_t n)
         rl_wait_vmcnt<0>();
 }
 
+// Block-table entries a caller has loaded ahead of attn_stream: lane l holds
+// entries first + l and first + 64 + l of table row `row` (0xFFFFFFFF: none
+// loaded; entries past the row's blocks are never used).
+struct TableWindow {
+    uint32_t win0 = 0, win1 = 0, row = 0xFFFFFFFFu, first = 0;
+};
+
 // The main loop of one wave: stream tiles [s_begin, s_end) of the row
 // sequence, starting in rollout start_b whose first tile is start_cum.
 // NS stages form a ring (stage k at st + k * st_stride; q slots at qs): while
@@ -500,7 +545,8 @@ __device__ __forceinline__ void wait_tiles(uint32_t n)
 template <int D, int G, int DT, int TPB, int NS, class CtxFn>
 __device__ __forceinline__ void attn_stream(const AttnParams &p, const CtxFn &cf, uint32_t wave_id, uint32_t s_begin,
                                             uint32_t s_end, uint32_t start_b, uint32_t start_cum,
-                                            RL_LDS uint8_t *st, uint32_t st_stride, RL_LDS uint8_t *qs, int lane)
+                                            RL_LDS uint8_t *st, uint32_t st_stride, RL_LDS uint8_t *qs, int lane,
+                                            const TableWindow &win = TableWindow{})
 {
     using C = Cfg<D, G, DT, TPB>;
     static_assert(NS >= 2 && NS <= 8, "stages");
@@ -516,9 +562,11 @@ __device__ __forceinline__ void attn_stream(const AttnParams &p, const CtxFn &cf
     is.left = s_end - s_begin;
     is.first = true;
     is.qcount = 0;
-    is.wrow = 0xFFFFFFFFu;
-    is.wfirst = 0;
-    is.win0 = is.win1 = 0;
+    is.wrow = win.row;
+    is.wfirst = win.first;
+    is.win0 = win.win0;
+    is.win1 = win.win1;
+    is.settle_window();
 
     RowState<D, G, DT, TPB> rs;
     StageMeta m[NS];  // indexed with compile-time slots only (the ring loop is unrolled)

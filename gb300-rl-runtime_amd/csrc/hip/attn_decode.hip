@@ -39,6 +39,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "attn_core.h"
 #include "kv_layout.h"
 #include "rl_dev_common.h"
@@ -58,6 +60,7 @@ namespace {
 struct SideSample {
     SampleParams sp;
     uint32_t attn_wgs;
+    uint32_t full_grid;  // the caller left the number of waves to the library (grid_waves 0)
 };
 
 // Stages of the per-wave tile ring. Two (one tile in flight while one is
@@ -223,6 +226,277 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p, AppendPar
     const uint32_t R0 = cum_b + g * nu;
     merge_row<D, G, DT, 256, GH>(p, b, g, h0, R0, nu, U, NW, bad, threadIdx.x, s_f, s_L);
 }
+
+// ---- few rows: workgroups of their own --------------------------------------------
+// A small batch is a chain of latencies: attn_decode_kernel's plan (the prefix
+// over the contexts, two barriers), table, tile, partials per wave, then a
+// merge that first finds its partials, up to 256 per row. Here the grid names
+// the row: RW waves of a workgroup stream contiguous shares of its tiles, the
+// table window is loaded beside the context, both stages' copies fly
+// (CtxRow), and the waves' partials are merged in the stage buffers they no
+// longer need. A row has one workgroup, and the step one launch, or up to
+// kRowsMaxSplit with one partial each for rows_merge_kernel.
+// Bound: latency, about 1 us per tile and wave (copy, then a chain of MFMAs
+// and cross-lane steps) and 2 us per launch; a row's KV comes through its
+// workgroups' compute units only, hence the rule at rows_split.
+// Measured, calls back to back (us, against attn_decode_kernel +
+// attn_merge_kernel; GQA 4, d128, bf16, with the append): 1 x 128 tokens
+// (without) 5.4 (10.2), 1 x 517 8.8 (12.9), 1 x 4,096 12.9 (31.9), 4 x
+// U[100, 1,024] 9.5 (15.4), 8 x U[512, 4,096] 23.2 (25.8), 32 x U[100, 200]
+// 10.8 (15.4); d64: 2 x U[64, 2,048] 9.2 (18.8).
+template <int D>
+constexpr int rows_waves_of()
+{
+    return D == 64 ? 16 : 8;
+}
+
+// Workgroups of a launch that are done with every KV read, counted in eight
+// groups of their own cache line and one counter above (an atomic on one
+// address takes about 30 ns, so 256 workgroups on one would queue). The last
+// workgroup of a group clears its counter and counts the group; the last
+// group's clears the top one. Launches on the library stream follow one
+// another, so every launch finds zeros.
+constexpr uint32_t kDoneGroups = 8;
+constexpr uint32_t kDoneStride = 32;  // counters 128 bytes apart
+__device__ uint32_t g_rows_done[(kDoneGroups + 1) * kDoneStride];
+
+__device__ __forceinline__ bool last_workgroup(uint32_t wg, uint32_t wgs)
+{
+    const uint32_t groups = wgs <= 2 * kDoneGroups ? 1u : kDoneGroups;  // (few workgroups: one counter)
+    const uint32_t grp = wg % groups, in_grp = (wgs - grp + groups - 1) / groups;
+    uint32_t *c = g_rows_done + grp * kDoneStride, *top = g_rows_done + kDoneGroups * kDoneStride;
+    if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != in_grp - 1)
+        return false;
+    __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (groups == 1)
+        return true;
+    if (__hip_atomic_fetch_add(top, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != groups - 1)
+        return false;
+    __hip_atomic_store(top, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+// The append of the whole batch by one workgroup. The step's contract is that
+// every context is read before any token is appended (a row may read a block
+// another row appends to), so the launch's last workgroup to finish its reads
+// appends for all. Writing after reads needs no cache maintenance: the reads
+// were complete before their workgroup counted itself.
+constexpr uint32_t kRowsAppendMax = 64;  // (rollout, kv head) rows one workgroup appends
+
+// Thread tid's 16-byte chunks of the batch's append (chunk tid + k nthr of
+// all rows' K and V, rows in (b, g) order): loaded and addressed before the
+// attention starts, stored by store() after it. Without a copy-on-write
+// source (those rows take append_row, one wave each).
+template <int N>
+struct AppendChunks {
+    uint8_t *dst[N];  // NULL: nothing to write
+    rl_u32x4 v[N];
+
+    __device__ __forceinline__ void load(const AppendParams &p, uint32_t rows, uint32_t tid, uint32_t nthr)
+    {
+        // (each loop's loads go out together)
+        const uint32_t chunks = p.row_bytes / 16, items = rows * 2 * chunks;
+        uint32_t at[N], b[N], trow[N], pos[N], blk[N];
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const uint32_t i = min(tid + k * nthr, items - 1);
+            const uint32_t r = i / (2 * chunks), plane = i / chunks % 2, c = i % chunks;
+            at[k] = plane * (p.token_count * p.row_bytes) + c * 16;
+            b[k] = r / p.kv_heads;
+            trow[k] = r;
+            pos[k] = p.positions[b[k]];
+            v[k] = *(const rl_u32x4 *)((plane ? p.v_new : p.k_new) + (size_t)r * p.row_bytes + c * 16);
+        }
+        if (p.row_map) {
+            uint32_t m[N];
+#pragma unroll
+            for (int k = 0; k < N; k++)
+                m[k] = p.row_map[b[k]];
+#pragma unroll
+            for (int k = 0; k < N; k++)
+                trow[k] += (m[k] - b[k]) * p.kv_heads;
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            blk[k] = p.table[(size_t)trow[k] * p.table_stride + min(pos[k] / p.token_count, p.table_stride - 1)];
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const bool ok = tid + k * nthr < items && pos[k] / p.token_count < p.table_stride &&
+                            blk[k] < p.arena_blocks;
+            dst[k] = ok ? p.arena + (uint64_t)blk[k] * p.block_bytes + at[k] + pos[k] % p.token_count * p.row_bytes
+                        : nullptr;
+        }
+    }
+
+    __device__ __forceinline__ void store() const
+    {
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            if (dst[k])
+                *(rl_u32x4 *)dst[k] = v[k];
+    }
+};
+
+// The append on its own, after the rows of a larger batch.
+__global__ __launch_bounds__(64) void rows_append_kernel(AppendParams p)
+{
+    append_row(p, blockIdx.y, blockIdx.x, threadIdx.x, 64);
+}
+
+// Merges the partials of a row's workgroups and appends its token. Workgroup
+// (x, b): 256 output elements of row (b, x / blocks per row); every load but
+// the append's table entry is addressed by the grid alone, so they go out
+// together.
+constexpr uint32_t kRowsMaxSplit = 32;
+
+template <int D, int G, int DT, int MS>
+__global__ __launch_bounds__(256) void rows_merge_kernel(AttnParams p, AppendParams ap)
+{
+    constexpr uint32_t RW = rows_waves_of<D>();
+    constexpr uint32_t PART = G * D + 2 * G, NE = G * D, BLK = (NE + 255) / 256;
+    const uint32_t g = blockIdx.x / BLK, b = blockIdx.y, row = b * p.kv_heads + g, S = p.nwaves;
+    const uint32_t e = blockIdx.x % BLK * 256 + threadIdx.x, ec = min(e, NE - 1);
+    const float *part = p.part + (size_t)row * S * PART;
+    const uint32_t cin = rl_sload(p.ctx + b);
+    float o[MS], mm[MS], ll[MS];
+#pragma unroll
+    for (uint32_t i = 0; i < MS; i++) {
+        const float *pp = part + (size_t)min(i, S - 1) * PART;
+        o[i] = pp[ec];
+        mm[i] = pp[NE + 2 * (ec / D)];
+        ll[i] = pp[NE + 2 * (ec / D) + 1];
+    }
+    if (ap.arena && blockIdx.x % BLK == 0 && threadIdx.x >= 192)
+        append_row(ap, b, g, threadIdx.x - 192, 64);
+    const uint32_t nu = tiles_of(p, cin);
+    const uint32_t n = (min(RW * S, nu) + RW - 1) / RW;  // workgroups of the row with tiles
+    if (n < 2 || e >= NE)
+        return;  // (one workgroup wrote the row itself)
+    float M = -INFINITY;
+#pragma unroll
+    for (uint32_t i = 0; i < MS; i++) {
+        mm[i] = i < n ? mm[i] : -INFINITY;
+        M = fmaxf(M, mm[i]);
+    }
+    float L = 0.f, O = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < MS; i++) {
+        const float f = mm[i] == -INFINITY ? 0.f : exp2f(mm[i] - M);
+        L = i < n ? fmaf(ll[i], f, L) : L;
+        O = i < n ? fmaf(o[i], f, O) : O;
+    }
+    float v = (L > 0.f || L != L) ? O / L : 0.f;
+    if (cin > p.max_ctx)
+        v = __builtin_nanf("");
+    const size_t at = ((size_t)b * p.q_heads + (size_t)g * G) * D + e;
+    if (p.out)
+        p.out[at] = rl_from_f32<DT>(v);
+    if (p.out_f32)
+        p.out_f32[at] = v;
+}
+
+template <int D, int G, int DT, int TPB>
+__global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(AttnParams p, AppendParams ap)
+{
+    using C = Cfg<D, G, DT, TPB>;
+    constexpr int RW = rows_waves_of<D>();
+    constexpr int NS = 2;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds_st[NS][RW * C::STAGE];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds_q[RW * NS * C::QSLOT];
+    static_assert(C::PART * 4 <= C::STAGE, "a partial fits the stage it replaces");
+
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wg = xcd_contiguous_wg(gridDim.x);
+    const uint32_t S = p.nwaves;  // workgroups per row
+    const uint32_t row = wg / S, s = wg % S;
+    const uint32_t b = row / p.kv_heads, g = row % p.kv_heads;
+    // the row's first 128 table entries, loaded beside its context (in bounds
+    // of the row whatever the context is)
+    TableWindow win;
+    win.row = table_row_of(p, b) * p.kv_heads + g;
+    const uint32_t *trow = p.table + (size_t)win.row * p.table_stride;
+    win.win0 = trow[min((uint32_t)lane, p.table_stride - 1)];
+    win.win1 = trow[min(64u + lane, p.table_stride - 1)];
+    const uint32_t cin = rl_sload(p.ctx + b);
+    constexpr int NCH = (int)(kRowsAppendMax * 2 * C::RB / 16 / (RW * 64));
+    AppendChunks<NCH> app;
+    const bool whole = ap.arena && !ap.cow_src;
+    if (whole)
+        app.load(ap, gridDim.x, threadIdx.x, RW * 64);
+    const bool bad = cin > p.max_ctx;
+    const uint32_t nu = tiles_of(p, cin);
+    const uint32_t nw = min(RW * S, nu);  // waves of the row with tiles, ...
+    const uint32_t first = s * RW;
+    const uint32_t mine = first < nw ? min((uint32_t)RW, nw - first) : 0u;  // ... and of this workgroup
+    if (wave < mine) {
+        // row_end's partial index (wave id + row) is 0: each wave's part is its
+        // own first stage
+        AttnParams pw = p;
+        RL_LDS uint8_t *st = (RL_LDS uint8_t *)lds_st[0] + wave * C::STAGE;
+        pw.part = (float *)(lds_st[0] + wave * C::STAGE);
+        const uint32_t R0 = g * nu, w = first + wave;
+        attn_stream<D, G, DT, TPB, NS>(pw, CtxRow{{cin}}, 0u - row, R0 + w * nu / nw, R0 + (w + 1) * nu / nw, b, 0u, st, RW * C::STAGE, (RL_LDS uint8_t *)lds_q + wave * NS * C::QSLOT, lane, win);
+    }
+    __syncthreads();
+    if (nu == 0) {
+        if (s == 0)
+            empty_row<D, G, DT, G>(p, b, g, 0, bad, threadIdx.x, RW * 64);
+    } else if (nw > 1 && mine) {
+        const bool whole_row = mine == nw;
+        const size_t obase = ((size_t)b * p.q_heads + (size_t)g * G) * D;
+        for (uint32_t e = threadIdx.x; e < (uint32_t)(G * D); e += RW * 64) {
+            const uint32_t h = e / D;
+            float o[RW], mm[RW], ll[RW], M = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < RW; i++) {
+                const float *part = (const float *)(lds_st[0] + min((uint32_t)i, mine - 1) * C::STAGE);
+                const bool ok = (uint32_t)i < mine;
+                o[i] = ok ? part[e] : 0.f;
+                mm[i] = ok ? part[G * D + 2 * h] : -INFINITY;
+                ll[i] = ok ? part[G * D + 2 * h + 1] : 0.f;
+                M = fmaxf(M, mm[i]);
+            }
+            float L = 0.f, O = 0.f;
+#pragma unroll
+            for (int i = 0; i < RW; i++) {
+                const float f = mm[i] == -INFINITY ? 0.f : exp2f(mm[i] - M);
+                L = fmaf(ll[i], f, L);
+                O = fmaf(o[i], f, O);
+            }
+            if (!whole_row) {  // a partial of this workgroup's tiles
+                float *part = p.part + (size_t)wg * C::PART;
+                part[e] = O;
+                if (e % D == 0) {
+                    part[G * D + 2 * h] = M;
+                    part[G * D + 2 * h + 1] = L;
+                }
+                continue;
+            }
+            float v = (L > 0.f || L != L) ? O / L : 0.f;
+            if (bad)
+                v = __builtin_nanf("");
+            if (p.out)
+                p.out[obase + e] = rl_from_f32<DT>(v);
+            if (p.out_f32)
+                p.out_f32[obase + e] = v;
+        }
+    }
+    if (!ap.arena)
+        return;
+    uint32_t *last = (uint32_t *)lds_q;  // (the q slots are free)
+    if (threadIdx.x == 0)
+        *last = last_workgroup(wg, gridDim.x);
+    __syncthreads();
+    if (!*last)
+        return;
+    if (whole) {
+        app.store();
+    } else {
+        for (uint32_t r = wave; r < gridDim.x; r += RW)
+            append_row(ap, r / ap.kv_heads, r % ap.kv_heads, lane, 64);
+    }
+}
 }  // namespace
 
 // ---- launcher ------------------------------------------------------------------
@@ -264,10 +538,69 @@ WsLayout ws_layout(const rl_attn_decode_args_t *a)
     return w;
 }
 
+// Workgroups per row for the rows kernel, or 0 when the batch is not its kind.
+// The rows' workgroups must fit the device once. One workgroup per row when
+// its waves take at most two tiles each of the longest context allowed (1 row
+// of 300 tokens: 8.2 us split in three, 9.3 whole at three tiles a wave), else
+// as many as there are compute units for, up to one tile per wave. Ragged
+// contexts leave the waves of short rows idle, where the even split of
+// attn_decode_kernel does not, so the rows kernel stops at 8 tiles per wave
+// (16 rollouts of up to 4,096: 39.6 us against 38.2), at 4 with d64 (24 of up
+// to 2,048 at 8 tiles: 19.1 against 18.9), at 16 up to 64 rows,
+// whose even split pays for merging up to 256 partials per row (2 rollouts of
+// up to 32,768: 45.0 against 54.9), and takes a lone rollout always (32,768:
+// 32.4 against 51.8).
+constexpr uint32_t kRowsWholeTiles = 2;
+
+template <int D>
+uint32_t rows_split(uint32_t batch, uint32_t kv_heads, uint32_t max_ctx)
+{
+    const uint64_t rows = (uint64_t)batch * kv_heads;
+    const uint32_t cus = rl_cu_count(), rw = rows_waves_of<D>();
+    if (rows > cus)
+        return 0;
+    const uint64_t tiles = std::max<uint64_t>(1, ((uint64_t)max_ctx + kTile - 1) / kTile);
+    if (tiles <= (uint64_t)rw * kRowsWholeTiles)
+        return 1;
+    const uint64_t most = std::min<uint64_t>(kRowsMaxSplit, cus / rows);
+    const uint64_t want = std::min<uint64_t>(most, (tiles + rw - 1) / rw);
+    const uint64_t limit = rows <= 64 ? 16 : D == 64 ? 4 : 8;
+    return batch == 1 || tiles <= rw * want * limit ? (uint32_t)want : 0;
+}
+
+template <int D, int G, int DT, int TPB>
+int launch_rows(AttnParams p, const AppendParams &ap, uint32_t split)
+{
+    const uint32_t rows = p.batch * p.kv_heads;
+    AppendParams in = ap;
+    if (split > 1 || rows > kRowsAppendMax)
+        in.arena = nullptr;
+    p.nwaves = split;
+    hipLaunchKernelGGL((attn_rows_kernel<D, G, DT, TPB>), dim3(rows * split), dim3(rows_waves_of<D>() * 64), 0,
+                       rl_stream(), p, in);
+    if (rl_check_launch("attn_rows_kernel launch"))
+        return -1;
+    if (split > 1) {
+        const dim3 grid(p.kv_heads * ((G * D + 255) / 256), p.batch);
+        if (split <= 8)
+            hipLaunchKernelGGL((rows_merge_kernel<D, G, DT, 8>), grid, dim3(256), 0, rl_stream(), p, ap);
+        else
+            hipLaunchKernelGGL((rows_merge_kernel<D, G, DT, kRowsMaxSplit>), grid, dim3(256), 0, rl_stream(), p, ap);
+        return rl_check_launch("rows_merge_kernel launch");
+    }
+    if (ap.arena == in.arena)
+        return 0;
+    hipLaunchKernelGGL(rows_append_kernel, dim3(p.kv_heads, p.batch), dim3(64), 0, rl_stream(), ap);
+    return rl_check_launch("rows_append_kernel launch");
+}
+
 template <int D, int G, int DT, int TPB>
 int launch(const AttnParams &p, const AppendParams &ap, SideSample ss)
 {
     using C = Cfg<D, G, DT, TPB>;
+    if (ss.full_grid && ss.sp.splits == 0)
+        if (const uint32_t split = rows_split<D>(p.batch, p.kv_heads, p.max_ctx))
+            return launch_rows<D, G, DT, TPB>(p, ap, split);
     const uint32_t wgs = (p.nwaves + C::W - 1) / C::W;
     ss.attn_wgs = wgs;
     const uint32_t slices = ss.sp.splits * ss.sp.rows;  // 0 without a side sampling
@@ -387,12 +720,14 @@ SideSample no_side()
     ss.sp.splits = 0;
     ss.sp.rows = 0;
     ss.attn_wgs = 0;
+    ss.full_grid = 0;
     return ss;
 }
 
 int attn_run(const rl_attn_decode_args_t *a, const AppendParams &ap, const uint32_t *row_map = nullptr,
-             const SideSample &ss = no_side())
+             SideSample ss = no_side())
 {
+    ss.full_grid = a->grid_waves == 0;
     const WsLayout w = ws_layout(a);
     if (!a->workspace || a->workspace_bytes < w.total) {
         rl_set_error("rl_hip_attn_decode: workspace %zu bytes < %zu required", a->workspace_bytes, w.total);
@@ -489,6 +824,11 @@ int rl_decode_step_greedy_side(const rl_attn_decode_args_t *attn, const rl_kv_ap
     const char *who = "rl_hip_decode_sample_step";
     if (append ? step_validate(attn, append, who) : (rl_require_open(who) || validate(attn)))
         return -1;
+    // few rows: rl_hip_attn_decode takes the rows kernel, whose results these must equal
+    const bool d128 = attn->layout.head_dim == 128;
+    if (attn->grid_waves == 0 && (d128 ? rows_split<128>(attn->batch, attn->kv_heads, attn->max_ctx)
+                                       : rows_split<64>(attn->batch, attn->kv_heads, attn->max_ctx)))
+        return 1;
     uint32_t splits = 0;
     size_t cand_off = 0;
     const int k = rl_sample_greedy_split(samp, &splits, &cand_off);

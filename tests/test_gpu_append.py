@@ -89,3 +89,77 @@ def test_decode_step_equals_attention_then_append(rl, gpu, orc, olib, dtype):
                        pos.ctypes.data, cow.ctypes.data, kn.ctypes.data, vn.ctypes.data)
     assert np.array_equal(arb, ref_arena)
     gh.check_attn(o16b.reshape(B, QH, D), o32b, orc.attn_f64(olib, w, 0 if dtype == "bf16" else 1), dtype)
+
+
+# the kernels for few rows: one workgroup per row with the append in the
+# launch (up to 64 rows) or after it, up to 8 and more workgroups per row
+@pytest.mark.parametrize("batch,qh,kvh,d,tpb,dtype,hi", [
+    (1, 32, 8, 128, 16, "bf16", 256), (3, 16, 8, 128, 16, "fp16", 200), (30, 8, 8, 64, 32, "bf16", 500),
+    (5, 32, 8, 64, 16, "fp16", 3000), (8, 64, 8, 128, 32, "bf16", 1500), (1, 8, 1, 128, 16, "bf16", 7000),
+    (7, 8, 8, 128, 16, "bf16", 129)])
+def test_few_rows_step(rl, gpu, orc, olib, batch, qh, kvh, d, tpb, dtype, hi):
+    """Ragged contexts (0, 1, tile edges, past max_ctx: NaN), a row that
+    appends into a block another row reads (every context is read first),
+    copy-on-write or none: rl_hip_decode_step three times over equals
+    rl_hip_attn_decode then rl_hip_kv_append byte for byte, the attention is
+    within the fp64 tolerance, the arena equals the oracle's append."""
+    import gpu_helpers as gh
+    import synth
+
+    print(f"[few rows] batch={batch} heads={qh}/{kvh} d={d} ctx<={hi}", flush=True)
+    rng = np.random.default_rng(batch + hi)
+    ctx = rng.integers(1, hi + 1, batch)
+    ctx[0] = hi
+    for i, c in enumerate((0, 1, 15, 16, 17)):
+        if i + 1 < batch:
+            ctx[i + 1] = c
+    w = synth.make_decode(7, batch, qh, kvh, d, 1, hi, dtype=dtype, token_count=tpb, ctx=ctx, max_ctx=hi, spare_blocks=8)
+    dt = rl.DTYPE_BF16 if dtype == "bf16" else rl.DTYPE_FP16
+    n = batch * qh * d
+    ref = orc.attn_f64(olib, w, 0 if dtype == "bf16" else 1)
+    over = w.ctx.copy()
+    if batch > 6:
+        over[6] = hi + 1                                      # beyond max_ctx: NaN outputs
+    pos, table2 = w.ctx.copy(), w.table.copy()
+    if batch > 2:
+        table2[2, :, 0], pos[2] = w.table[0, :, 0], 3         # into the first block row 0 reads
+    n_used = w.arena.size // w.block_bytes - 8
+    for cow_on in (False, True):
+        cow = np.full((batch, kvh), -1, np.int32)
+        cow[::2] = n_used + rng.integers(0, 8, cow[::2].shape)
+        kn = rng.integers(0, 256, (batch, kvh, d * 2), dtype=np.uint8)
+        vn = rng.integers(0, 256, (batch, kvh, d * 2), dtype=np.uint8)
+        layout = rl.KvLayoutDesc.paged(tpb, d)
+        res = []
+        for fused in (False, True, True, True):
+            bufs = {k: rl.DeviceBuffer.from_array(v) for k, v in
+                    (("arena", w.arena), ("table", w.table), ("table2", table2), ("ctx", over), ("q", w.q),
+                     ("pos", pos), ("cow", cow), ("kn", kn), ("vn", vn))}
+            out, out32 = rl.DeviceBuffer(n * 2), rl.DeviceBuffer(n * 4)
+            a = rl.attn_args(bufs["arena"], layout, bufs["table"], w.table_stride, batch, qh, kvh, dt, bufs["ctx"], hi,
+                             bufs["q"], out, out32)
+            ws = rl.attn_workspace(a)
+            ap = rl.AppendArgs(arena_base=bufs["arena"].ptr, arena_bytes=bufs["arena"].nbytes, layout=layout,
+                               block_table=bufs["table2"].ptr, table_stride=w.table_stride, batch=batch, kv_heads=kvh,
+                               positions=bufs["pos"].ptr, cow_src=bufs["cow"].ptr if cow_on else None,
+                               k_new=bufs["kn"].ptr, v_new=bufs["vn"].ptr)
+            if fused:
+                rl.decode_step(a, ap)
+            else:
+                rl.attn_decode(a)
+                rl.kv_append(ap)
+            rl.sync()
+            res.append((out.download(np.uint16, n), out32.download(np.uint32, n),
+                        bufs["arena"].download(np.uint8, w.arena.size)))
+            for b in list(bufs.values()) + [out, out32, ws]:
+                b.close()
+        for r in res[1:]:
+            assert all(np.array_equal(x, y) for x, y in zip(r, res[0]))
+        want = w.arena.copy()
+        olib.orc_kv_append(want.ctypes.data, w.block_bytes, tpb, d * 2, table2.ctypes.data, w.table_stride, batch, kvh,
+                           pos.ctypes.data, cow.ctypes.data if cow_on else None, kn.ctypes.data, vn.ctypes.data)
+        assert np.array_equal(res[0][2], want)
+        o16, o32 = res[0][0].reshape(batch, qh, d), res[0][1].view(np.float32).reshape(batch, qh, d)
+        keep = np.arange(batch) != 6 if batch > 6 else np.ones(batch, bool)
+        assert batch <= 6 or np.isnan(o32[6]).all()
+        gh.check_attn(o16[keep], o32[keep], ref[keep], dtype)
