@@ -529,13 +529,6 @@ __device__ __forceinline__ void wait_tiles(uint32_t n)
         rl_wait_vmcnt<0>();
 }
 
-// Block-table entries a caller has loaded ahead of attn_stream: lane l holds
-// entries first + l and first + 64 + l of table row `row` (0xFFFFFFFF: none
-// loaded; entries past the row's blocks are never used).
-struct TableWindow {
-    uint32_t win0 = 0, win1 = 0, row = 0xFFFFFFFFu, first = 0;
-};
-
 // The main loop of one wave: stream tiles [s_begin, s_end) of the row
 // sequence, starting in rollout start_b whose first tile is start_cum.
 // NS stages form a ring (stage k at st + k * st_stride; q slots at qs): while
@@ -545,8 +538,7 @@ struct TableWindow {
 template <int D, int G, int DT, int TPB, int NS, class CtxFn>
 __device__ __forceinline__ void attn_stream(const AttnParams &p, const CtxFn &cf, uint32_t wave_id, uint32_t s_begin,
                                             uint32_t s_end, uint32_t start_b, uint32_t start_cum,
-                                            RL_LDS uint8_t *st, uint32_t st_stride, RL_LDS uint8_t *qs, int lane,
-                                            const TableWindow &win = TableWindow{})
+                                            RL_LDS uint8_t *st, uint32_t st_stride, RL_LDS uint8_t *qs, int lane)
 {
     using C = Cfg<D, G, DT, TPB>;
     static_assert(NS >= 2 && NS <= 8, "stages");
@@ -562,11 +554,9 @@ __device__ __forceinline__ void attn_stream(const AttnParams &p, const CtxFn &cf
     is.left = s_end - s_begin;
     is.first = true;
     is.qcount = 0;
-    is.wrow = win.row;
-    is.wfirst = win.first;
-    is.win0 = win.win0;
-    is.win1 = win.win1;
-    is.settle_window();
+    is.wrow = 0xFFFFFFFFu;
+    is.wfirst = 0;
+    is.win0 = is.win1 = 0;
 
     RowState<D, G, DT, TPB> rs;
     StageMeta m[NS];  // indexed with compile-time slots only (the ring loop is unrolled)

@@ -194,13 +194,20 @@ constexpr int merge_heads_of()
     return G >= 2 ? G / 2 : 1;
 }
 
+// (the append has a wave of its own, the fifth: its chain of loads runs beside
+// the merge's and not before it. 16 rollouts of 8 KV heads: 37.8 -> 36.3 us
+// for the step; with 2,048 rows, eight workgroups to a compute unit, the wave
+// cost more than it hid, 137.8 -> 139.0, and the fourth wave appends.)
+constexpr int kMergeThreads5 = 320;
+constexpr uint32_t kMergeRows5 = 1024;  // at most as many rows take the fifth wave
+
 template <int D, int G, int DT, int HS>
-__global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p, AppendParams ap, SideSample ss)
+__global__ __launch_bounds__(kMergeThreads5) void attn_merge_kernel(AttnParams p, AppendParams ap, SideSample ss)
 {
     constexpr int GH = G / HS;
     if (blockIdx.y >= p.batch) {  // greedy rows of the sampling riding in this launch, one wave each
         const uint32_t r = ((blockIdx.y - p.batch) * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
-        if (r < ss.sp.rows)
+        if (threadIdx.x < 256 && r < ss.sp.rows)
             greedy_merge_row(ss.sp, r, (int)(threadIdx.x & 63), true);
         return;
     }
@@ -214,7 +221,12 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p, AppendPar
     const uint32_t cin = rl_sload(p.ctx + b);
     const uint32_t U = rl_sload(p.cum + p.batch);
     const uint32_t cum_b = rl_sload(p.cum + b);
-    if (ap.arena && h0 == 0 && threadIdx.x >= 192)
+    if (threadIdx.x >= 256) {
+        if (h0 == 0)
+            append_row(ap, b, g, threadIdx.x - 256, 64);
+        return;
+    }
+    if (ap.arena && h0 == 0 && blockDim.x == 256 && threadIdx.x >= 192)
         append_row(ap, b, g, threadIdx.x - 192, 64);
     const bool bad = cin > p.max_ctx;
     const uint32_t nu = tiles_of(p, cin);
@@ -231,10 +243,9 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p, AppendPar
 // A small batch is a chain of latencies: attn_decode_kernel's plan (the prefix
 // over the contexts, two barriers), table, tile, partials per wave, then a
 // merge that first finds its partials, up to 256 per row. Here the grid names
-// the row: RW waves of a workgroup stream contiguous shares of its tiles, the
-// table window is loaded beside the context, both stages' copies fly
-// (CtxRow), and the waves' partials are merged in the stage buffers they no
-// longer need. A row has one workgroup, and the step one launch, or up to
+// the row: RW waves of a workgroup stream contiguous shares of its tiles,
+// both stages' copies fly (CtxRow), and the waves' partials are merged in the
+// stage buffers they no longer need. A row has one workgroup, and the step one launch, or up to
 // kRowsMaxSplit with one partial each for rows_merge_kernel.
 // Bound: latency, about 1 us per tile and wave (copy, then a chain of MFMAs
 // and cross-lane steps) and 2 us per launch; a row's KV comes through its
@@ -307,25 +318,26 @@ struct AppendChunks {
             pos[k] = p.positions[b[k]];
             v[k] = *(const rl_u32x4 *)((plane ? p.v_new : p.k_new) + (size_t)r * p.row_bytes + c * 16);
         }
+        // a position past the table (a row that appends nothing) reads neither
+        // the row map nor the table
+        bool ok[N];
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            ok[k] = tid + k * nthr < items && pos[k] / p.token_count < p.table_stride;
         if (p.row_map) {
-            uint32_t m[N];
 #pragma unroll
             for (int k = 0; k < N; k++)
-                m[k] = p.row_map[b[k]];
-#pragma unroll
-            for (int k = 0; k < N; k++)
-                trow[k] += (m[k] - b[k]) * p.kv_heads;
+                if (ok[k])
+                    trow[k] += (p.row_map[b[k]] - b[k]) * p.kv_heads;
         }
 #pragma unroll
         for (int k = 0; k < N; k++)
-            blk[k] = p.table[(size_t)trow[k] * p.table_stride + min(pos[k] / p.token_count, p.table_stride - 1)];
+            blk[k] = ok[k] ? p.table[(size_t)trow[k] * p.table_stride + pos[k] / p.token_count] : 0u;
 #pragma unroll
-        for (int k = 0; k < N; k++) {
-            const bool ok = tid + k * nthr < items && pos[k] / p.token_count < p.table_stride &&
-                            blk[k] < p.arena_blocks;
-            dst[k] = ok ? p.arena + (uint64_t)blk[k] * p.block_bytes + at[k] + pos[k] % p.token_count * p.row_bytes
-                        : nullptr;
-        }
+        for (int k = 0; k < N; k++)
+            dst[k] = ok[k] && blk[k] < p.arena_blocks
+                         ? p.arena + (uint64_t)blk[k] * p.block_bytes + at[k] + pos[k] % p.token_count * p.row_bytes
+                         : nullptr;
     }
 
     __device__ __forceinline__ void store() const
@@ -350,11 +362,16 @@ __global__ __launch_bounds__(64) void rows_append_kernel(AppendParams p)
 constexpr uint32_t kRowsMaxSplit = 32;
 
 template <int D, int G, int DT, int MS>
-__global__ __launch_bounds__(256) void rows_merge_kernel(AttnParams p, AppendParams ap)
+__global__ __launch_bounds__(kMergeThreads5) void rows_merge_kernel(AttnParams p, AppendParams ap)
 {
     constexpr uint32_t RW = rows_waves_of<D>();
     constexpr uint32_t PART = G * D + 2 * G, NE = G * D, BLK = (NE + 255) / 256;
     const uint32_t g = blockIdx.x / BLK, b = blockIdx.y, row = b * p.kv_heads + g, S = p.nwaves;
+    if (threadIdx.x >= 256) {
+        if (blockIdx.x % BLK == 0)
+            append_row(ap, b, g, threadIdx.x - 256, 64);
+        return;
+    }
     const uint32_t e = blockIdx.x % BLK * 256 + threadIdx.x, ec = min(e, NE - 1);
     const float *part = p.part + (size_t)row * S * PART;
     const uint32_t cin = rl_sload(p.ctx + b);
@@ -366,8 +383,6 @@ __global__ __launch_bounds__(256) void rows_merge_kernel(AttnParams p, AppendPar
         mm[i] = pp[NE + 2 * (ec / D)];
         ll[i] = pp[NE + 2 * (ec / D) + 1];
     }
-    if (ap.arena && blockIdx.x % BLK == 0 && threadIdx.x >= 192)
-        append_row(ap, b, g, threadIdx.x - 192, 64);
     const uint32_t nu = tiles_of(p, cin);
     const uint32_t n = (min(RW * S, nu) + RW - 1) / RW;  // workgroups of the row with tiles
     if (n < 2 || e >= NE)
@@ -411,13 +426,6 @@ __global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(Attn
     const uint32_t S = p.nwaves;  // workgroups per row
     const uint32_t row = wg / S, s = wg % S;
     const uint32_t b = row / p.kv_heads, g = row % p.kv_heads;
-    // the row's first 128 table entries, loaded beside its context (in bounds
-    // of the row whatever the context is)
-    TableWindow win;
-    win.row = table_row_of(p, b) * p.kv_heads + g;
-    const uint32_t *trow = p.table + (size_t)win.row * p.table_stride;
-    win.win0 = trow[min((uint32_t)lane, p.table_stride - 1)];
-    win.win1 = trow[min(64u + lane, p.table_stride - 1)];
     const uint32_t cin = rl_sload(p.ctx + b);
     constexpr int NCH = (int)(kRowsAppendMax * 2 * C::RB / 16 / (RW * 64));
     AppendChunks<NCH> app;
@@ -436,7 +444,7 @@ __global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(Attn
         RL_LDS uint8_t *st = (RL_LDS uint8_t *)lds_st[0] + wave * C::STAGE;
         pw.part = (float *)(lds_st[0] + wave * C::STAGE);
         const uint32_t R0 = g * nu, w = first + wave;
-        attn_stream<D, G, DT, TPB, NS>(pw, CtxRow{{cin}}, 0u - row, R0 + w * nu / nw, R0 + (w + 1) * nu / nw, b, 0u, st, RW * C::STAGE, (RL_LDS uint8_t *)lds_q + wave * NS * C::QSLOT, lane, win);
+        attn_stream<D, G, DT, TPB, NS>(pw, CtxRow{{cin}}, 0u - row, R0 + w * nu / nw, R0 + (w + 1) * nu / nw, b, 0u, st, RW * C::STAGE, (RL_LDS uint8_t *)lds_q + wave * NS * C::QSLOT, lane);
     }
     __syncthreads();
     if (nu == 0) {
@@ -582,10 +590,11 @@ int launch_rows(AttnParams p, const AppendParams &ap, uint32_t split)
         return -1;
     if (split > 1) {
         const dim3 grid(p.kv_heads * ((G * D + 255) / 256), p.batch);
+        const uint32_t threads = ap.arena ? kMergeThreads5 : 256;
         if (split <= 8)
-            hipLaunchKernelGGL((rows_merge_kernel<D, G, DT, 8>), grid, dim3(256), 0, rl_stream(), p, ap);
+            hipLaunchKernelGGL((rows_merge_kernel<D, G, DT, 8>), grid, dim3(threads), 0, rl_stream(), p, ap);
         else
-            hipLaunchKernelGGL((rows_merge_kernel<D, G, DT, kRowsMaxSplit>), grid, dim3(256), 0, rl_stream(), p, ap);
+            hipLaunchKernelGGL((rows_merge_kernel<D, G, DT, kRowsMaxSplit>), grid, dim3(threads), 0, rl_stream(), p, ap);
         return rl_check_launch("rows_merge_kernel launch");
     }
     if (ap.arena == in.arena)
@@ -614,12 +623,13 @@ int launch(const AttnParams &p, const AppendParams &ap, SideSample ss)
     // workgroup in extra grid rows.
     constexpr int HS = merge_heads_of<G>();
     const bool hs = HS > 1 && (uint64_t)p.nwaves >= 8ull * p.batch * p.kv_heads;
+    const uint32_t threads = ap.arena && p.batch * p.kv_heads <= kMergeRows5 ? kMergeThreads5 : 256;
     const uint32_t gx = hs ? p.kv_heads * HS : p.kv_heads;
     const uint32_t gy = p.batch + (slices ? (ss.sp.rows + 4 * gx - 1) / (4 * gx) : 0u);
     if (hs)
-        hipLaunchKernelGGL((attn_merge_kernel<D, G, DT, HS>), dim3(gx, gy), dim3(256), 0, rl_stream(), p, ap, ss);
+        hipLaunchKernelGGL((attn_merge_kernel<D, G, DT, HS>), dim3(gx, gy), dim3(threads), 0, rl_stream(), p, ap, ss);
     else
-        hipLaunchKernelGGL((attn_merge_kernel<D, G, DT, 1>), dim3(gx, gy), dim3(256), 0, rl_stream(), p, ap, ss);
+        hipLaunchKernelGGL((attn_merge_kernel<D, G, DT, 1>), dim3(gx, gy), dim3(threads), 0, rl_stream(), p, ap, ss);
     return rl_check_launch("attn_merge_kernel launch");
 }
 
@@ -795,6 +805,12 @@ extern "C" int rl_hip_decode_step(const rl_attn_decode_args_t *attn, const rl_kv
     return attn_run(attn, append_params(append));
 }
 
+bool rl_attn_few_rows(const rl_attn_decode_args_t *a)
+{
+    return a->grid_waves == 0 && (a->layout.head_dim == 128 ? rows_split<128>(a->batch, a->kv_heads, a->max_ctx)
+                                                            : rows_split<64>(a->batch, a->kv_heads, a->max_ctx)) > 0;
+}
+
 int rl_attn_check(const rl_attn_decode_args_t *a)
 {
     return validate(a);
@@ -825,9 +841,7 @@ int rl_decode_step_greedy_side(const rl_attn_decode_args_t *attn, const rl_kv_ap
     if (append ? step_validate(attn, append, who) : (rl_require_open(who) || validate(attn)))
         return -1;
     // few rows: rl_hip_attn_decode takes the rows kernel, whose results these must equal
-    const bool d128 = attn->layout.head_dim == 128;
-    if (attn->grid_waves == 0 && (d128 ? rows_split<128>(attn->batch, attn->kv_heads, attn->max_ctx)
-                                       : rows_split<64>(attn->batch, attn->kv_heads, attn->max_ctx)))
+    if (rl_attn_few_rows(attn))
         return 1;
     uint32_t splits = 0;
     size_t cand_off = 0;

@@ -41,6 +41,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "rl_hip.h"
 #include "rl_hip_internal.h"
 #include "attn_core.h"
@@ -362,9 +364,12 @@ __global__ __launch_bounds__(kFThreads) void decode_fused_kernel(FusedParams f)
 
 // Combines the partials of every row split across pieces (merge_span), writes
 // rows without tiles and appends the step's K/V token (the row's first
-// workgroup). HS workgroups of G / HS heads per row, as attn_merge_kernel.
+// workgroup, by a fifth wave launched only with an append). HS workgroups of
+// G / HS heads per row, as attn_merge_kernel.
+constexpr int kPieceMergeThreads = 320;
+
 template <int D, int G, int DT, int HS>
-__global__ __launch_bounds__(256) void merge_pieces_kernel(AttnParams p, AppendParams ap, const SplitIn *psi)
+__global__ __launch_bounds__(kPieceMergeThreads) void merge_pieces_kernel(AttnParams p, AppendParams ap, const SplitIn *psi)
 {
     constexpr int GH = G / HS;
     __shared__ float s_f[kMergeLds * G];
@@ -375,8 +380,11 @@ __global__ __launch_bounds__(256) void merge_pieces_kernel(AttnParams p, AppendP
     const uint32_t cin = rl_sload(p.ctx + b);
     const uint32_t U = rl_sload(p.cum + p.batch);
     const uint32_t cum_b = rl_sload(p.cum + b);
-    if (ap.arena && h0 == 0 && threadIdx.x >= 192)
-        append_row(ap, b, g, threadIdx.x - 192, 64);
+    if (threadIdx.x >= 256) {
+        if (h0 == 0)
+            append_row(ap, b, g, threadIdx.x - 256, 64);
+        return;
+    }
     const bool bad = cin > p.max_ctx;
     const uint32_t nu = tiles_of(p, cin);
     if (nu == 0) {
@@ -982,11 +990,12 @@ int launch(int what, const FusedParams &f, const AppendParams &ap, hipStream_t s
             // holds (16 at two output elements per thread) take workgroups of
             // two heads, as attn_merge_kernel
             const uint64_t rows = (uint64_t)f.p.batch * f.p.kv_heads;
+            const dim3 threads(ap.arena ? kPieceMergeThreads : 256);
             if (HS > 1 && (uint64_t)f.si.wgs * kFWaves >= 16ull * rows)
-                hipLaunchKernelGGL((merge_pieces_kernel<D, G, DT, HS>), dim3(f.p.kv_heads * HS, f.p.batch), dim3(256),
-                                   0, stream, f.p, ap, (const SplitIn *)f.si_out);
+                hipLaunchKernelGGL((merge_pieces_kernel<D, G, DT, HS>), dim3(f.p.kv_heads * HS, f.p.batch), threads, 0,
+                                    stream, f.p, ap, (const SplitIn *)f.si_out);
             else
-                hipLaunchKernelGGL((merge_pieces_kernel<D, G, DT, 1>), dim3(f.p.kv_heads, f.p.batch), dim3(256), 0,
+                hipLaunchKernelGGL((merge_pieces_kernel<D, G, DT, 1>), dim3(f.p.kv_heads, f.p.batch), threads, 0,
                                    stream, f.p, ap, (const SplitIn *)f.si_out);
             if (rl_check_launch("merge_pieces_kernel launch"))
                 return -1;
@@ -1103,6 +1112,35 @@ AppendParams append_or_none(const rl_kv_append_args_t *append)
 
 }  // namespace
 
+namespace {
+
+// Fused-kernel shapes whose step is faster as the decode step and then the
+// sampling, each in its own kernels:
+//  - rows without top-k above 32,768 logits, which a sampling workgroup would
+//    stream twice from one compute unit and rl_hip_sample spreads over slices
+//    (64 rollouts of U[512, 4,096], 128,256 logits, top-p: 163 us against 179;
+//    200 of U[100, 1,000], 60,000 logits: 141 against 252);
+//  - batches of few rows (rl_attn_few_rows) with rows of 16,384 logits and
+//    more, bound by latency (4 x U[100, 1,000] with 32,000 logits, top-k 50:
+//    23.8 us against 26.9; 2 x U[1,000, 8,000], 128,256 logits: 33.2 against
+//    53.5; but 1 x U[100, 300] with 4,000 logits 13.8 against 12.7).
+// The caller's workspace decides whether they can: one sized for other
+// sampling arguments keeps the fused kernel. So does the ring-driven step,
+// whose launched and self-scheduled forms sample with the same code.
+bool one_after_the_other(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp)
+{
+    const bool no_topk = !samp->top_k && (samp->top_k_all == 0 || samp->top_k_all >= samp->vocab);
+    return (no_topk && !samp->greedy && samp->vocab > RL_ROW_SAMPLER_VOCAB) ||
+           (samp->vocab >= 16384 && rl_attn_few_rows(attn));
+}
+
+size_t apart_ws(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp)
+{
+    return (rl_hip_attn_decode_workspace(attn) + 255) / 256 * 256 + rl_hip_sample_workspace(samp);
+}
+
+}  // namespace
+
 extern "C" size_t rl_hip_decode_sample_step_workspace(const rl_attn_decode_args_t *attn,
                                                       const rl_sample_args_t *samp)
 {
@@ -1110,10 +1148,10 @@ extern "C" size_t rl_hip_decode_sample_step_workspace(const rl_attn_decode_args_
         return 0;
     const size_t fused = fused_ws(attn, split_in_of(attn, samp)).total;
     // the shapes outside the fused kernel run the two steps one after the other
-    const size_t a = rl_hip_attn_decode_workspace(attn);
-    const size_t s = rl_hip_sample_workspace(samp);
-    const size_t split = (a + 255) / 256 * 256 + s;
-    return fused_eligible(attn) ? fused : split;
+    const size_t split = apart_ws(attn, samp);
+    if (!fused_eligible(attn))
+        return split;
+    return one_after_the_other(attn, samp) ? std::max(fused, split) : fused;
 }
 
 namespace {
@@ -1183,12 +1221,13 @@ int decode_sample_step_rows(const rl_attn_decode_args_t *attn, const rl_kv_appen
 {
     if (fused_validate(attn, append, samp, who))
         return -1;
-    const size_t need = rl_hip_decode_sample_step_workspace(attn, samp);
+    const bool fused = fused_eligible(attn);
+    const size_t need = fused ? fused_ws(attn, split_in_of(attn, samp)).total : apart_ws(attn, samp);
     if (!workspace || workspace_bytes < need) {
         rl_set_error("%s: workspace %zu bytes < %zu required", who, workspace_bytes, need);
         return -1;
     }
-    if (!fused_eligible(attn)) {
+    if (!fused || (!row_map && one_after_the_other(attn, samp) && workspace_bytes >= apart_ws(attn, samp))) {
         // One decode step (or the attention alone), then the sampling, on
         // the library stream. A greedy batch that the sampler splits rides
         // in the attention's two launches instead: its slices as workgroups

@@ -40,6 +40,11 @@ int rl_decode_sample_step_mapped(const rl_attn_decode_args_t *attn, const rl_kv_
 int rl_attn_check(const rl_attn_decode_args_t *a);
 int rl_decode_step_check(const rl_attn_decode_args_t *attn, const rl_kv_append_args_t *append, const char *who);
 int rl_sample_check(const rl_sample_args_t *a);
+// Whether rl_hip_attn_decode takes its kernels for few rows (attn_decode.hip).
+bool rl_attn_few_rows(const rl_attn_decode_args_t *a);
+// The longest rows without top-k that one workgroup samples from registers;
+// longer ones are spread over slices (sample.hip).
+#define RL_ROW_SAMPLER_VOCAB 32768u
 // For a greedy batch (a->greedy set) that rl_hip_sample runs as split +
 // merge: 1, with the slices per row and the offset of the candidate lists in
 // its workspace (the slice records start at 0); 0 when the batch takes

@@ -278,6 +278,7 @@ __global__ __launch_bounds__(kMergeThreads) void sample_stream_kernel(SamplePara
 // whole-row path above, which reads it again from memory.
 constexpr int kRowRounds = 16;
 constexpr uint32_t kRowVocab = (uint32_t)kMergeWaves * kRowRounds * 256u;  // 32,768
+static_assert(kRowVocab == RL_ROW_SAMPLER_VOCAB, "the decode step's route goes by it");
 constexpr int kRowBins = 8192;
 constexpr int kRowPer = kRowBins / kMergeThreads;  // bins per thread in the scan
 constexpr int kRowList = 256;

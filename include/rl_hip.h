@@ -608,7 +608,10 @@ int rl_hip_decode_step(const rl_attn_decode_args_t *attn, const rl_kv_append_arg
  * and the sampling without a KV append. Shapes whose tiles do not fit the
  * fused kernel's LDS (GQA groups of 8 at head_dim 128, batches above 1,024)
  * run rl_hip_decode_step (rl_hip_attn_decode without an append) and then
- * rl_hip_sample on the same workspace, with exactly their results. */
+ * rl_hip_sample on the same workspace, with exactly their results; so do, as
+ * long as the workspace was sized for them, samplings without top-k of more
+ * than 32,768 logits and batches of few rows with 16,384 logits or more,
+ * which are faster that way. */
 size_t rl_hip_decode_sample_step_workspace(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp);
 int rl_hip_decode_sample_step(const rl_attn_decode_args_t *attn, const rl_kv_append_args_t *append,
                               const rl_sample_args_t *samp, void *workspace, size_t workspace_bytes);
@@ -620,11 +623,11 @@ int rl_hip_decode_sample_step(const rl_attn_decode_args_t *attn, const rl_kv_app
  * its K/V token (prev_attn / prev_append, partials in prev_workspace, which
  * that step was given as its workspace). So the rows of attn are complete
  * only after the next step (or rl_hip_decode_pipeline_flush) has run; rows
- * that one piece covered are written at once. Tokens, logprobs and the
- * appended KV equal rl_hip_decode_sample_step's; the attention is its fp32
- * math (bit for bit when the split is the same, as at the first step: the
- * merge work of the sampling waves shifts the split otherwise), within 1e-4
- * of fp64. prev_attn NULL: nothing to merge (the first step). The two micro-batches alternate, each with its own
+ * that one piece covered are written at once. Tokens and the appended KV
+ * equal rl_hip_decode_sample_step's, and so do the logprobs (to fp32 rounding
+ * where that call runs its two steps apart); the attention is its fp32 math
+ * (bit for bit when the split is the same, as at the first step: the merge
+ * work of the sampling waves shifts the split otherwise), within 1e-4 of fp64. prev_attn NULL: nothing to merge (the first step). The two micro-batches alternate, each with its own
  * workspace of rl_hip_decode_sample_step_workspace bytes; prev_attn must
  * have attn's heads, dtype and layout, and prev_append must not write what
  * attn reads (the other micro-batch's blocks; a slot at or past a row's

@@ -590,3 +590,42 @@ def test_fused_greedy_rides_in_the_attention(rl, gpu, orc, olib):
     assert np.array_equal(lp.download(np.float32, R).view(np.uint32), res[0][4].view(np.uint32))
     for b in (lg, tok, lp, sws):
         b.close()
+
+
+@pytest.mark.parametrize("batch,hi,rows,vocab,samp", [
+    (40, 900, 40, 40000, dict(temperature=0.9, top_k=0, top_p=0.9, seed=4, step=2)),
+    (70, 300, 9, 32772, dict(temperature=1.0, top_k=0, top_p=1.0, seed=5, step=3)),
+    (3, 700, 3, 16384, dict(temperature=0.8, top_k=50, top_p=0.9, seed=6, step=4)),
+    (1, 5000, 17, 32000, dict(temperature=1.0, top_k=0, top_p=0.9, seed=7, step=5))])
+def test_steps_one_after_the_other(rl, gpu, orc, olib, batch, hi, rows, vocab, samp):
+    """Fused-kernel shapes that run as the decode step and then the sampling
+    (long rows without top-k, few rows): against the oracle, and on a
+    workspace of the fused kernel's own size, which keeps that kernel."""
+    rng = np.random.default_rng(vocab + batch)
+    w = synth.make_decode(61, batch, 32, 8, 128, 1, hi, max_ctx=hi)
+    kn, vn = _kv_rows(rng, w)
+    logits = rng.standard_normal((rows, vocab), dtype=np.float32)
+    want, wlp = orc.sample_rows(olib, logits, False, samp["temperature"], samp["top_k"], samp["top_p"], samp["seed"],
+                                samp["step"])
+    res = _run(rl, w, hi, w.ctx.copy(), None, kn, vn, logits, **samp)
+    _check(orc, olib, w, hi, w.ctx.copy(), None, kn, vn, logits, res, want, wlp)
+    layout = rl.KvLayoutDesc.paged(16, 128)
+    bufs = {k: rl.DeviceBuffer.from_array(v) for k, v in
+            (("arena", w.arena), ("table", w.table), ("ctx", w.ctx), ("q", w.q), ("logits", logits))}
+    n = batch * 32 * 128
+    out, out32, tok, lp = (rl.DeviceBuffer(k) for k in (n * 2, n * 4, rows * 4, rows * 4))
+    a = rl.attn_args(bufs["arena"], layout, bufs["table"], w.table_stride, batch, 32, 8, rl.DTYPE_BF16, bufs["ctx"],
+                     hi, bufs["q"], out, out32)
+    s = rl.sample_args(bufs["logits"], rows, vocab, vocab, tok, lp, **samp)
+    full = rl.decode_sample_step_workspace_bytes(a, s)
+    a.grid_waves, s.greedy = 64, 1            # arguments that the fused kernel takes whatever the sizes
+    ws = rl.DeviceBuffer(rl.decode_sample_step_workspace_bytes(a, s))
+    a.grid_waves, s.greedy = 0, 0
+    assert ws.nbytes <= full
+    rl.decode_sample_step(a, None, s, ws)
+    rl.sync()
+    assert np.array_equal(tok.download(np.uint32, rows), want)
+    o32 = out32.download(np.float32, (batch, 32, 128))
+    assert (gh.rownorm_err(o32, orc.attn_f64(olib, w, 0)) < 1e-4).all()
+    for b in list(bufs.values()) + [out, out32, tok, lp, ws]:
+        b.close()
