@@ -1141,16 +1141,19 @@ size_t apart_ws(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp)
 
 }  // namespace
 
+size_t rl_step_workspace_mapped(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp)
+{
+    return fused_eligible(attn) ? fused_ws(attn, split_in_of(attn, samp)).total : apart_ws(attn, samp);
+}
+
 extern "C" size_t rl_hip_decode_sample_step_workspace(const rl_attn_decode_args_t *attn,
                                                       const rl_sample_args_t *samp)
 {
     if (rl_require_open("rl_hip_decode_sample_step_workspace") || rl_attn_check(attn) || rl_sample_check(samp))
         return 0;
-    const size_t fused = fused_ws(attn, split_in_of(attn, samp)).total;
     // the shapes outside the fused kernel run the two steps one after the other
     const size_t split = apart_ws(attn, samp);
-    if (!fused_eligible(attn))
-        return split;
+    const size_t fused = rl_step_workspace_mapped(attn, samp);
     return one_after_the_other(attn, samp) ? std::max(fused, split) : fused;
 }
 
@@ -1222,7 +1225,7 @@ int decode_sample_step_rows(const rl_attn_decode_args_t *attn, const rl_kv_appen
     if (fused_validate(attn, append, samp, who))
         return -1;
     const bool fused = fused_eligible(attn);
-    const size_t need = fused ? fused_ws(attn, split_in_of(attn, samp)).total : apart_ws(attn, samp);
+    const size_t need = rl_step_workspace_mapped(attn, samp);
     if (!workspace || workspace_bytes < need) {
         rl_set_error("%s: workspace %zu bytes < %zu required", who, workspace_bytes, need);
         return -1;
@@ -1299,7 +1302,7 @@ int pipeline_step_on(hipStream_t stream, const rl_attn_decode_args_t *attn, cons
         rl_set_error("%s: the shape does not fit the fused kernel (use rl_hip_decode_sample_step)", who);
         return -1;
     }
-    const size_t need = rl_hip_decode_sample_step_workspace(attn, samp);
+    const size_t need = rl_step_workspace_mapped(attn, samp);
     if (!workspace || workspace_bytes < need) {
         rl_set_error("%s: workspace %zu bytes < %zu required", who, workspace_bytes, need);
         return -1;

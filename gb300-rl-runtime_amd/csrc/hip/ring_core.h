@@ -450,9 +450,9 @@ inline int ring_layout(const rl_ring_step_args_t *a, RingWs &w)
     w.step = w.rstep + up256(B * 8);
     rl_attn_decode_args_t t = attn_of(a, nullptr, 0);
     rl_sample_args_t s = samp_of(a);
-    w.step_bytes = rl_hip_decode_sample_step_workspace(&t, &s);
-    if (w.step_bytes == 0)
+    if (rl_require_open("rl_hip_ring_step_workspace") || rl_attn_check(&t) || rl_sample_check(&s))
         return -1;
+    w.step_bytes = rl_step_workspace_mapped(&t, &s);
     size_t o = w.step + up256(w.step_bytes);
     for (RingWs::Set &x : w.set) {
         x.rmap = o;

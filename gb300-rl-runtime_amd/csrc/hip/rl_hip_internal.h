@@ -34,6 +34,11 @@ int rl_attn_mapped(const rl_attn_decode_args_t *attn, const uint32_t *row_map);
 int rl_decode_sample_step_mapped(const rl_attn_decode_args_t *attn, const rl_kv_append_args_t *append,
                                  const rl_sample_args_t *samp, const uint32_t *row_map, void *workspace,
                                  size_t workspace_bytes, const char *who);
+// The workspace of that mapped form and of the pipelined step, for checked
+// arguments: rl_hip_decode_sample_step_workspace without the room that call
+// may use to run its two steps apart, so the same whatever is sampled for the
+// shapes of the fused kernel.
+size_t rl_step_workspace_mapped(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp);
 
 // Argument checks of the attention, the decode step and the sampler (0, or
 // -1 with the error set), for entry points that combine them.

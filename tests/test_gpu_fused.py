@@ -627,5 +627,9 @@ def test_steps_one_after_the_other(rl, gpu, orc, olib, batch, hi, rows, vocab, s
     assert np.array_equal(tok.download(np.uint32, rows), want)
     o32 = out32.download(np.float32, (batch, 32, 128))
     assert (gh.rownorm_err(o32, orc.attn_f64(olib, w, 0)) < 1e-4).all()
+    tok.upload(np.zeros(rows, np.uint32))     # the pipelined form needs no more than that workspace either
+    rl.decode_pipeline_step(a, s, ws)
+    rl.sync()
+    assert np.array_equal(tok.download(np.uint32, rows), want)
     for b in list(bufs.values()) + [out, out32, tok, lp, ws]:
         b.close()
