@@ -443,8 +443,12 @@ __global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(Attn
         AttnParams pw = p;
         RL_LDS uint8_t *st = (RL_LDS uint8_t *)lds_st[0] + wave * C::STAGE;
         pw.part = (float *)(lds_st[0] + wave * C::STAGE);
-        const uint32_t R0 = g * nu, w = first + wave;
-        attn_stream<D, G, DT, TPB, NS>(pw, CtxRow{{cin}}, 0u - row, R0 + w * nu / nw, R0 + (w + 1) * nu / nw, b, 0u, st, RW * C::STAGE, (RL_LDS uint8_t *)lds_q + wave * NS * C::QSLOT, lane);
+        const uint32_t R0 = g * nu;
+        // (a row of 2^23 tiles and more times its wave count exceeds 32 bits)
+        const uint64_t w = first + wave;
+        attn_stream<D, G, DT, TPB, NS>(pw, CtxRow{{cin}}, 0u - row, R0 + (uint32_t)(w * nu / nw),
+                                       R0 + (uint32_t)((w + 1) * nu / nw), b, 0u, st, RW * C::STAGE,
+                                       (RL_LDS uint8_t *)lds_q + wave * NS * C::QSLOT, lane);
     }
     __syncthreads();
     if (nu == 0) {

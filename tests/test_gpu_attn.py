@@ -123,3 +123,35 @@ def test_guards_poison_instead_of_faulting(rl, gpu, orc, olib):
     out16, out32 = gh.run_attn(rl, w, max_ctx=100)
     assert np.isnan(out32[1]).all() and np.isnan(out32[2, 4:8]).all()
     assert np.isfinite(out32[0]).all() and np.isfinite(out32[2, :4]).all()
+
+
+def test_lone_rollout_beyond_32_bit_products(rl, gpu):
+    """One rollout of 2^24 + 1 tiles: a wave's share times the number of tiles
+    needs more than 32 bits. Every table entry names the same block, so the
+    result is the attention over that block's 16 tokens. Tolerance: each of
+    256 waves per row adds up to 65,537 equal fp32 terms one after another, to
+    the weight sum and to the output, at most 65,537 * 2^-24 relative each."""
+    tiles, kvh, d = (1 << 24) + 1, 8, 128
+    print(f"[attn] B=1 heads={kvh} d={d} tiles={tiles}", flush=True)
+    w = synth.make_decode(77, 1, kvh, kvh, d, 16, 16)
+    assert w.arena.size >= w.block_bytes and w.table_stride >= 1
+    blk = int(w.table[0, 0, 0])
+    layout = rl.KvLayoutDesc.paged(16, d)
+    arena = rl.DeviceBuffer.from_array(w.arena[blk * w.block_bytes:(blk + 1) * w.block_bytes].copy())
+    table = rl.DeviceBuffer(kvh * tiles * 4, zero=True)
+    ctx = rl.DeviceBuffer.from_array(np.array([tiles * 16], np.uint32))
+    q = rl.DeviceBuffer.from_array(w.q)
+    out, out32 = rl.DeviceBuffer(kvh * d * 2), rl.DeviceBuffer(kvh * d * 4)
+    a = rl.attn_args(arena, layout, table, tiles, 1, kvh, kvh, rl.DTYPE_BF16, ctx, tiles * 16, q, out, out32)
+    ws = rl.attn_workspace(a)
+    rl.attn_decode(a)
+    rl.sync()
+    got = out32.download(np.float32, (kvh, d)).astype(np.float64)
+    kv = synth.from_scalar16(w.arena[blk * w.block_bytes:(blk + 1) * w.block_bytes].view(np.uint16), "bf16")
+    k, v = kv.astype(np.float64).reshape(2, 16, d)
+    x = synth.from_scalar16(w.q.reshape(kvh, d), "bf16").astype(np.float64) @ k.T / np.sqrt(d)
+    p = np.exp(x - x.max(-1, keepdims=True))
+    want = p @ v / p.sum(-1, keepdims=True)
+    assert (gh.rownorm_err(got, want) < 2 * 65537 * 2.0 ** -24 + 1e-4).all()
+    for b in (arena, table, ctx, q, out, out32, ws):
+        b.close()
