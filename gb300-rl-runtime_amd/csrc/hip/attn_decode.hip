@@ -194,15 +194,13 @@ constexpr int merge_heads_of()
     return G >= 2 ? G / 2 : 1;
 }
 
-// (the append has a wave of its own, the fifth: its chain of loads runs beside
-// the merge's and not before it. 16 rollouts of 8 KV heads: 37.8 -> 36.3 us
-// for the step; with 2,048 rows, eight workgroups to a compute unit, the wave
-// cost more than it hid, 137.8 -> 139.0, and the fourth wave appends.)
-constexpr int kMergeThreads5 = 320;
-constexpr uint32_t kMergeRows5 = 1024;  // at most as many rows take the fifth wave
-
-template <int D, int G, int DT, int HS>
-__global__ __launch_bounds__(kMergeThreads5) void attn_merge_kernel(AttnParams p, AppendParams ap, SideSample ss)
+// (THREADS 320: the fifth wave appends and does nothing else, while the
+// merge's workgroups are few, rl_append_wave; 256: the fourth appends before
+// it merges. Two kernels, for the registers: one that could do both needed 129
+// in the fused step's merge at group 4, past the 128 that leave a SIMD four
+// waves.)
+template <int D, int G, int DT, int HS, int THREADS>
+__global__ __launch_bounds__(THREADS) void attn_merge_kernel(AttnParams p, AppendParams ap, SideSample ss)
 {
     constexpr int GH = G / HS;
     if (blockIdx.y >= p.batch) {  // greedy rows of the sampling riding in this launch, one wave each
@@ -221,13 +219,15 @@ __global__ __launch_bounds__(kMergeThreads5) void attn_merge_kernel(AttnParams p
     const uint32_t cin = rl_sload(p.ctx + b);
     const uint32_t U = rl_sload(p.cum + p.batch);
     const uint32_t cum_b = rl_sload(p.cum + b);
-    if (threadIdx.x >= 256) {
-        if (h0 == 0)
-            append_row(ap, b, g, threadIdx.x - 256, 64);
-        return;
-    }
-    if (ap.arena && h0 == 0 && blockDim.x == 256 && threadIdx.x >= 192)
+    if constexpr (THREADS > 256) {
+        if (threadIdx.x >= 256) {
+            if (h0 == 0)
+                append_row(ap, b, g, threadIdx.x - 256, 64);
+            return;
+        }
+    } else if (ap.arena && h0 == 0 && threadIdx.x >= 192) {
         append_row(ap, b, g, threadIdx.x - 192, 64);
+    }
     const bool bad = cin > p.max_ctx;
     const uint32_t nu = tiles_of(p, cin);
     if (nu == 0) {
@@ -627,13 +627,20 @@ int launch(const AttnParams &p, const AppendParams &ap, SideSample ss)
     // workgroup in extra grid rows.
     constexpr int HS = merge_heads_of<G>();
     const bool hs = HS > 1 && (uint64_t)p.nwaves >= 8ull * p.batch * p.kv_heads;
-    const uint32_t threads = ap.arena && p.batch * p.kv_heads <= kMergeRows5 ? kMergeThreads5 : 256;
     const uint32_t gx = hs ? p.kv_heads * HS : p.kv_heads;
+    const bool wave = ap.arena && rl_append_wave((uint64_t)gx * p.batch);
     const uint32_t gy = p.batch + (slices ? (ss.sp.rows + 4 * gx - 1) / (4 * gx) : 0u);
-    if (hs)
-        hipLaunchKernelGGL((attn_merge_kernel<D, G, DT, HS>), dim3(gx, gy), dim3(threads), 0, rl_stream(), p, ap, ss);
+    auto run = [&](auto kernel, uint32_t threads) {
+        hipLaunchKernelGGL(kernel, dim3(gx, gy), dim3(threads), 0, rl_stream(), p, ap, ss);
+    };
+    if (hs && wave)
+        run(attn_merge_kernel<D, G, DT, HS, kMergeThreads5>, kMergeThreads5);
+    else if (hs)
+        run(attn_merge_kernel<D, G, DT, HS, 256>, 256);
+    else if (wave)
+        run(attn_merge_kernel<D, G, DT, 1, kMergeThreads5>, kMergeThreads5);
     else
-        hipLaunchKernelGGL((attn_merge_kernel<D, G, DT, 1>), dim3(gx, gy), dim3(threads), 0, rl_stream(), p, ap, ss);
+        run(attn_merge_kernel<D, G, DT, 1, 256>, 256);
     return rl_check_launch("attn_merge_kernel launch");
 }
 

@@ -364,12 +364,9 @@ __global__ __launch_bounds__(kFThreads) void decode_fused_kernel(FusedParams f)
 
 // Combines the partials of every row split across pieces (merge_span), writes
 // rows without tiles and appends the step's K/V token (the row's first
-// workgroup, by a fifth wave launched only with an append). HS workgroups of
-// G / HS heads per row, as attn_merge_kernel.
-constexpr int kPieceMergeThreads = 320;
-
-template <int D, int G, int DT, int HS>
-__global__ __launch_bounds__(kPieceMergeThreads) void merge_pieces_kernel(AttnParams p, AppendParams ap, const SplitIn *psi)
+// workgroup; THREADS and HS as in attn_merge_kernel).
+template <int D, int G, int DT, int HS, int THREADS>
+__global__ __launch_bounds__(THREADS) void merge_pieces_kernel(AttnParams p, AppendParams ap, const SplitIn *psi)
 {
     constexpr int GH = G / HS;
     __shared__ float s_f[kMergeLds * G];
@@ -380,10 +377,14 @@ __global__ __launch_bounds__(kPieceMergeThreads) void merge_pieces_kernel(AttnPa
     const uint32_t cin = rl_sload(p.ctx + b);
     const uint32_t U = rl_sload(p.cum + p.batch);
     const uint32_t cum_b = rl_sload(p.cum + b);
-    if (threadIdx.x >= 256) {
-        if (h0 == 0)
-            append_row(ap, b, g, threadIdx.x - 256, 64);
-        return;
+    if constexpr (THREADS > 256) {
+        if (threadIdx.x >= 256) {
+            if (h0 == 0)
+                append_row(ap, b, g, threadIdx.x - 256, 64);
+            return;
+        }
+    } else if (ap.arena && h0 == 0 && threadIdx.x >= 192) {
+        append_row(ap, b, g, threadIdx.x - 192, 64);
     }
     const bool bad = cin > p.max_ctx;
     const uint32_t nu = tiles_of(p, cin);
@@ -990,13 +991,20 @@ int launch(int what, const FusedParams &f, const AppendParams &ap, hipStream_t s
             // holds (16 at two output elements per thread) take workgroups of
             // two heads, as attn_merge_kernel
             const uint64_t rows = (uint64_t)f.p.batch * f.p.kv_heads;
-            const dim3 threads(ap.arena ? kPieceMergeThreads : 256);
-            if (HS > 1 && (uint64_t)f.si.wgs * kFWaves >= 16ull * rows)
-                hipLaunchKernelGGL((merge_pieces_kernel<D, G, DT, HS>), dim3(f.p.kv_heads * HS, f.p.batch), threads, 0,
-                                    stream, f.p, ap, (const SplitIn *)f.si_out);
+            const bool hs = HS > 1 && (uint64_t)f.si.wgs * kFWaves >= 16ull * rows;
+            const dim3 grid(hs ? f.p.kv_heads * HS : f.p.kv_heads, f.p.batch);
+            const bool wave = ap.arena && rl_append_wave((uint64_t)grid.x * grid.y);
+            auto run = [&](auto kernel, uint32_t threads) {
+                hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, f.p, ap, (const SplitIn *)f.si_out);
+            };
+            if (hs && wave)
+                run(merge_pieces_kernel<D, G, DT, HS, kMergeThreads5>, kMergeThreads5);
+            else if (hs)
+                run(merge_pieces_kernel<D, G, DT, HS, 256>, 256);
+            else if (wave)
+                run(merge_pieces_kernel<D, G, DT, 1, kMergeThreads5>, kMergeThreads5);
             else
-                hipLaunchKernelGGL((merge_pieces_kernel<D, G, DT, 1>), dim3(f.p.kv_heads, f.p.batch), threads, 0,
-                                   stream, f.p, ap, (const SplitIn *)f.si_out);
+                run(merge_pieces_kernel<D, G, DT, 1, 256>, 256);
             if (rl_check_launch("merge_pieces_kernel launch"))
                 return -1;
         }

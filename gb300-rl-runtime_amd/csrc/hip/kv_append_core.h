@@ -88,6 +88,19 @@ __device__ __forceinline__ void append_row(const AppendParams &p, uint32_t b, ui
     }
 }
 
+constexpr int kMergeThreads5 = 320;
+
+// Whether a merge kernel of `workgroups` workgroups (four waves each) gets a
+// fifth wave for the append, whose chain of loads then runs beside the
+// merge's. Up to two workgroups per compute unit it does: the step with
+// contexts of U[65, 114] takes, without and with it, 14.84 and 14.43 us at
+// 384 rows of GQA group 4, 15.33 and 14.81 at 512 (13.71 and 13.73, 14.51 and
+// 14.54 at group 1), and the fused step of 64 rollouts 27.3 and 26.1. Beyond,
+// the larger workgroups no longer all fit at once: 18.34 and 18.86 at 768
+// rows, 17.68 and 18.74 at group 1, 18.98 and 21.20 at 952 of group 1; fused
+// 41.0 and 43.9 at 1,024, 70.8 and 75.0 at 2,048.
+inline bool rl_append_wave(uint64_t workgroups) { return workgroups <= 2ull * rl_cu_count(); }
+
 // Host-side checks of an append's arguments (0 or -1 with the error set).
 inline int append_validate(const rl_kv_append_args_t *a, const char *who)
 {

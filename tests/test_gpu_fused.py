@@ -592,6 +592,23 @@ def test_fused_greedy_rides_in_the_attention(rl, gpu, orc, olib):
         b.close()
 
 
+@pytest.mark.parametrize("heads", [32, 64])
+@pytest.mark.parametrize("batch", [64, 65])
+def test_step_append_wave(rl, gpu, orc, olib, batch, heads):
+    """The append on a wave of its own (up to two merge workgroups per compute
+    unit, 512 rows) and on a merging wave (above), in the fused step and, at
+    GQA group 8, in the decode step; copy-on-write for some rows."""
+    rng = np.random.default_rng(batch + heads)
+    w = synth.make_decode(batch, batch, heads, 8, 128, 1, 200, max_ctx=200, spare_blocks=8)
+    cow = np.full((batch, 8), -1, np.int32)
+    cow[::5] = w.arena.size // w.block_bytes - 8 + rng.integers(0, 8, cow[::5].shape)
+    kn, vn = _kv_rows(rng, w)
+    logits = rng.standard_normal((4, 1000), dtype=np.float32)
+    want, wlp = orc.sample_rows(olib, logits, False, 0.9, 20, 0.9, 4, 2)
+    res = _run(rl, w, 200, w.ctx.copy(), cow, kn, vn, logits, temperature=0.9, top_k=20, top_p=0.9, seed=4, step=2)
+    _check(orc, olib, w, 200, w.ctx.copy(), cow, kn, vn, logits, res, want, wlp)
+
+
 @pytest.mark.parametrize("batch,hi,rows,vocab,samp", [
     (40, 900, 40, 40000, dict(temperature=0.9, top_k=0, top_p=0.9, seed=4, step=2)),
     (70, 300, 9, 32772, dict(temperature=1.0, top_k=0, top_p=1.0, seed=5, step=3)),
