@@ -410,6 +410,17 @@ __global__ __launch_bounds__(kMergeThreads5) void rows_merge_kernel(AttnParams p
         p.out_f32[at] = v;
 }
 
+// First tile of wave w of the nw (at most RW kRowsMaxSplit) that share a row
+// of nu tiles. The product exceeds 32 bits for rows of 2^23 tiles and more; a
+// 64-bit division on every row would cost 0.1 us of 7.6.
+template <int RW>
+__device__ __forceinline__ uint32_t wave_share(uint32_t w, uint32_t nu, uint32_t nw)
+{
+    if (nu < 0xFFFFFFFFu / (RW * kRowsMaxSplit))
+        return w * nu / nw;
+    return (uint32_t)((uint64_t)w * nu / nw);
+}
+
 template <int D, int G, int DT, int TPB>
 __global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(AttnParams p, AppendParams ap)
 {
@@ -443,11 +454,9 @@ __global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(Attn
         AttnParams pw = p;
         RL_LDS uint8_t *st = (RL_LDS uint8_t *)lds_st[0] + wave * C::STAGE;
         pw.part = (float *)(lds_st[0] + wave * C::STAGE);
-        const uint32_t R0 = g * nu;
-        // (a row of 2^23 tiles and more times its wave count exceeds 32 bits)
-        const uint64_t w = first + wave;
-        attn_stream<D, G, DT, TPB, NS>(pw, CtxRow{{cin}}, 0u - row, R0 + (uint32_t)(w * nu / nw),
-                                       R0 + (uint32_t)((w + 1) * nu / nw), b, 0u, st, RW * C::STAGE,
+        const uint32_t R0 = g * nu, w = first + wave;
+        attn_stream<D, G, DT, TPB, NS>(pw, CtxRow{{cin}}, 0u - row, R0 + wave_share<RW>(w, nu, nw),
+                                       R0 + wave_share<RW>(w + 1, nu, nw), b, 0u, st, RW * C::STAGE,
                                        (RL_LDS uint8_t *)lds_q + wave * NS * C::QSLOT, lane);
     }
     __syncthreads();
