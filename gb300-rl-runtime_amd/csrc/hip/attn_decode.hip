@@ -265,8 +265,11 @@ constexpr int rows_waves_of()
 // groups of their own cache line and one counter above (an atomic on one
 // address takes about 30 ns, so 256 workgroups on one would queue). The last
 // workgroup of a group clears its counter and counts the group; the last
-// group's clears the top one. Launches on the library stream follow one
-// another, so every launch finds zeros.
+// group's clears the top one. One set per device serves every caller because
+// only launches that follow one another use it: those made directly on the
+// library's one stream. A step recorded into a graph, which may be replayed
+// on any stream beside others, appends in a second launch (launch_rows), as
+// every other route of a step does. So each launch finds zeros.
 constexpr uint32_t kDoneGroups = 8;
 constexpr uint32_t kDoneStride = 32;  // counters 128 bytes apart
 __device__ uint32_t g_rows_done[(kDoneGroups + 1) * kDoneStride];
@@ -593,9 +596,18 @@ template <int D, int G, int DT, int TPB>
 int launch_rows(AttnParams p, const AppendParams &ap, uint32_t split)
 {
     const uint32_t rows = p.batch * p.kv_heads;
+    // The append in the launch itself: for steps whose launches are ordered by
+    // the library stream (g_rows_done); not while it is captured.
     AppendParams in = ap;
-    if (split > 1 || rows > kRowsAppendMax)
+    if (split > 1 || rows > kRowsAppendMax) {
         in.arena = nullptr;
+    } else if (ap.arena) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (rl_check_hip(hipStreamIsCapturing(rl_stream(), &st), "hipStreamIsCapturing"))
+            return -1;
+        if (st != hipStreamCaptureStatusNone)
+            in.arena = nullptr;
+    }
     p.nwaves = split;
     hipLaunchKernelGGL((attn_rows_kernel<D, G, DT, TPB>), dim3(rows * split), dim3(rows_waves_of<D>() * 64), 0,
                        rl_stream(), p, in);
@@ -918,6 +930,11 @@ int rl_attn_scratch_setup(int device)
                      kScratchDevices);
         return -1;
     }
+    // (no launch of an earlier session is left: rl_hip_close waits)
+    void *done = nullptr;
+    if (rl_check_hip(hipGetSymbolAddress(&done, HIP_SYMBOL(g_rows_done)), "hipGetSymbolAddress(g_rows_done)") ||
+        rl_check_hip(hipMemset(done, 0, sizeof(g_rows_done)), "hipMemset(g_rows_done)"))
+        return -1;
     if (g_scratch_dev[device])
         return 0;
     void *p = nullptr;
