@@ -572,9 +572,16 @@ WsLayout ws_layout(const rl_attn_decode_args_t *a)
 // (16 rollouts of up to 4,096: 39.6 us against 38.2), at 4 with d64 (24 of up
 // to 2,048 at 8 tiles: 19.1 against 18.9), at 16 up to 64 rows,
 // whose even split pays for merging up to 256 partials per row (2 rollouts of
-// up to 32,768: 45.0 against 54.9), and takes a lone rollout always (32,768:
-// 32.4 against 51.8).
+// up to 32,768: 45.0 against 54.9). A lone rollout takes it always when its
+// rows fill the device (8 KV heads: 32,768 tokens 32.4 against 51.8, 524,288
+// 370 against 382). With fewer KV heads it streams through fewer compute
+// units, but the even split then merges up to 2,048 partials per row in one
+// workgroup, so the rows kernel stops only at 1,024 tiles per wave (1, 2 and 4
+// KV heads: 131,072 tokens 45 against 1,011, 53 against 530 and 62 against
+// 303; 4,194,304, the limit, 1,238 against 1,364, 1,337 against 1,309 and
+// 1,588 against 1,724; 1 KV head at 8,388,608 2,462 against 1,897).
 constexpr uint32_t kRowsWholeTiles = 2;
+constexpr uint32_t kRowsLoneTiles = 1024;
 
 template <int D>
 uint32_t rows_split(uint32_t batch, uint32_t kv_heads, uint32_t max_ctx)
@@ -589,7 +596,8 @@ uint32_t rows_split(uint32_t batch, uint32_t kv_heads, uint32_t max_ctx)
     const uint64_t most = std::min<uint64_t>(kRowsMaxSplit, cus / rows);
     const uint64_t want = std::min<uint64_t>(most, (tiles + rw - 1) / rw);
     const uint64_t limit = rows <= 64 ? 16 : D == 64 ? 4 : 8;
-    return batch == 1 || tiles <= rw * want * limit ? (uint32_t)want : 0;
+    const bool lone = batch == 1 && (rows * want >= cus || tiles <= rw * want * kRowsLoneTiles);
+    return lone || tiles <= rw * want * limit ? (uint32_t)want : 0;
 }
 
 template <int D, int G, int DT, int TPB>
