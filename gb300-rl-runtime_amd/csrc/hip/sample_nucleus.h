@@ -10,30 +10,38 @@
 // from L2 / Infinity Cache. Every sum is of integers, so the token does not
 // depend on the split.
 //
-//  sample_split_kernel     slice maxima and exp sums (sample_core.h)
+//  nucleus_split_kernel    slice maxima and exp sums (split_slice of
+//                          sample_core.h); the row's histograms cleared
 //  nucleus_weigh_kernel    the row maximum m, then w = rl_sample_weight(x - m):
-//                          per bin of d = m - x (kNucBins over kBinSpan, a
-//                          monotone map, so a bin is a run of the (x desc,
-//                          index asc) order) when the row has a nucleus, per
-//                          round of 256 elements when it has none
+//                          added up per bin of d = m - x (kNucBins over
+//                          nuc_scale's span, a monotone map, so a bin is a run
+//                          of the (x desc, index asc) order) when the row has
+//                          a nucleus, per round of 256 elements when it has
+//                          none
 //  nucleus_edge_kernel     the bin where the cumulative weight reaches
-//                          thr = ceil(p W) (every slice's workgroup adds the
-//                          row's histograms up itself: 4 KiB a slice, less
-//                          than another launch costs); per round, the weight
-//                          in the bins above it; that bin's members
-//  nucleus_pick_kernel     the boundary member among them, the round where the
-//                          cumulative weight first exceeds the draw, and the
-//                          element in it
-// A row whose boundary bin holds more members than the lists take (massive
-// ties), or whose maximum is not finite, takes the exact whole-row path in
-// the last kernel.
+//                          thr = ceil(p W); per round, the weight in the bins
+//                          above it; that bin's members, listed per slice and
+//                          added up per sub-bin (1/kNucBins of the bin)
+//  nucleus_pick_kernel     the sub-bin where thr is reached and the boundary
+//                          member in it, the round where the cumulative weight
+//                          first exceeds the draw, and the element in it
+// A slice whose members exceed its list is read again in the last kernel. A
+// row whose boundary sub-bin holds more than one member per thread (ties), or
+// whose maximum is not finite, takes the exact whole-row path there.
 // Measured, calls back to back, against split + exact path (us): 37 x 128,256
-// at top-p 0.95 34.8 against 104.3 (the four kernels 4.5, 7.9, 13.2 and 9.2);
-// 256 rows 118 against 127; 512 x 131,072 217 against 250; 1 x 50,257 19.4
-// against 46.4; 64 x 128,256 at top-p 1 (no edge pass) 22.5 against 97.1.
-// Bound: vector-ALU issue in the weigh and edge passes (18 instructions of
-// weight per element, 4 cycles each), launch and dependent-load latency in
-// the pick. So the weights are not computed before the histograms arrive
+// ~N(0, 1) at top-p 0.95 33.6 against 104.4 (the four kernels 5.2, 9.9, 11.9
+// and 8.3), ~N(0, 0.3^2) at 0.9 33.0 against 107.9; 256 rows of those 112
+// against 130; 64 x 262,144 ~N(0, 1) at 0.9 65.6 against 206, 64 x 524,288 118
+// against 400; 512 x 131,072 203 against 250; 1 x 50,257 20.3 against 47.1; 64 x
+// 128,256 at top-p 1 (no edge pass) 22.4 against 97.2; 37 x 128,256 ~N(0,
+// 0.05^2) under five logits of 8 (every slice read again in the pick) 82
+// against 685 (there the radix search).
+// Bound: vector-ALU issue in the edge pass, 56 instructions a logit: 6.9 of its
+// 11.9 us over the whole device, 9 on a compute unit with three of the 592
+// workgroups; 5.0 of 9.9 us in the weigh pass (41 a logit), whose rest is the
+// histogram's LDS atomics (0.13 conflict cycles a logit) and the device-wide
+// ones. Launch and dependent-load latency in the pick, whose waves wait 70% of
+// their cycles. So the weights are not computed before the histograms arrive
 // (13.2 -> 14.1 us: more registers, no less issue).
 #pragma once
 
@@ -44,23 +52,31 @@ namespace {
 constexpr int kNucBins = kMergeThreads;                // 512: one bin per thread
 constexpr int kNucRounds = kSplitLen / 256;            // 32 rounds of 256 elements per slice
 constexpr int kNucWaveRounds = kNucRounds / kMergeWaves;
-constexpr int kNucMembers = 480;                       // boundary-bin members per slice
-constexpr int kNucRowMembers = 2048;                   // ... and per row, in LDS
-constexpr int kNucSubBins = kMergeThreads;
+constexpr int kNucMembers = 480;                       // boundary-bin members a slice lists
 constexpr uint32_t kNucXcds = 8;
+constexpr uint32_t kNucLast = 32;
 
-// A slice's part of the workspace, in place of its candidate list.
+// A slice's part of the workspace, in place of its candidate list. A row's
+// weights are added up in two of its slices' records, by one device-wide
+// atomic per bin and slice: per bin in slice 0's hist, per sub-bin of the
+// boundary bin in slice 1's (these rows have five slices and more). So the
+// later passes read 4 KiB a workgroup whatever the number of slices; each
+// slice with its own histogram, and the edge pass adding them up, took 35.5
+// us against 33.1 at 37 x 128,256 and reads slices^2 of them a row.
 struct NucSlice {
     unsigned long long hist[kNucBins];
     unsigned long long rounds[kNucRounds];
     uint32_t members;           // in the boundary bin (> kNucMembers: not all listed)
     uint32_t bstar;             // slice 0: the row's boundary bin, ...
     unsigned long long above;   // ... the weight in the bins above it
-    unsigned long long thr;     // ... and the nucleus threshold
+    unsigned long long thr;     // ... the nucleus threshold
+    float scale;                // ... and its bins per unit of d (nuc_scale)
+    uint32_t pad;
     uint2 list[kNucMembers];    // (bits of x, index)
 };
 static_assert(sizeof(NucSlice) <= kCandStride * sizeof(uint2), "a slice's record fits its candidate list");
 static_assert(kCandStride * sizeof(uint2) % 16 == 0, "records stay 16-byte aligned");
+static_assert(RL_ROW_SAMPLER_VOCAB >= kSplitLen, "longer rows have a slice 1");
 
 __device__ __forceinline__ NucSlice *nuc_slice(const SampleParams &p, uint32_t row, uint32_t split)
 {
@@ -82,21 +98,53 @@ __device__ __forceinline__ bool nuc_place(const SampleParams &p, uint32_t &split
 
 __device__ __forceinline__ bool nuc_trunc(float topp) { return topp > 0.f && topp < 1.f; }
 
-// The row maximum from the slices' records (splits <= 64: one per lane).
-__device__ __forceinline__ float nuc_row_max(const SampleParams &p, uint32_t row, int lane)
+// The row maximum and the sum of exp(x - max) from the slices' records
+// (splits <= 64: one per lane).
+__device__ __forceinline__ void nuc_row(const SampleParams &p, uint32_t row, int lane, float &m, float &z)
 {
-    float mx = -INFINITY;
-    if ((uint32_t)lane < p.splits)
+    float mx = -INFINITY, zs = 0.f;
+    if ((uint32_t)lane < p.splits) {
         mx = p.stats[(size_t)row * p.splits + lane].max_x;
-    return wave_max(mx);
+        zs = p.stats[(size_t)row * p.splits + lane].sum_exp;
+    }
+    m = wave_max(mx);
+    z = wave_sum(mx == -INFINITY ? 0.f : zs * exp2f((mx - m) * 1.4426950408889634f));
 }
 
-// Bin coordinate of x and the bin of a coordinate: monotone in x.
-__device__ __forceinline__ float nuc_t(float m, float x) { return (m - x) * ((float)kNucBins / kBinSpan); }
+// Bins per unit of d. The elements past d = D weigh at most V e^-D together,
+// which is below the (1 - p) z outside the nucleus from D = ln(V / ((1 - p) z))
+// on: the bins span that much (an eighth more, for the roundings) and the last
+// one takes the rest, so that they are as narrow as the row's spread allows
+// (128,256 logits ~N(0, 0.3^2) at p 0.9 span 3.7: 800 members in the boundary
+// bin, 3,600 with a span of 17 for every row).
+__device__ __forceinline__ float nuc_scale(float z, uint32_t vocab, float topp)
+{
+    const float span = fminf(logf((float)vocab / (z * (1.0f - topp))) + 0.125f, kBinSpan);
+    return (float)(kNucBins - 1) / fmaxf(span, 0.125f);
+}
+
+// Bin coordinate of x, the bin of a coordinate and the sub-bin of a coordinate
+// in bin b: all monotone in x (t - b is exact or monotone, and the factor a
+// power of two).
+__device__ __forceinline__ float nuc_t(float m, float x, float scale) { return (m - x) * scale; }
 
 __device__ __forceinline__ uint32_t nuc_bin(float t)
 {
     return t < (float)(kNucBins - 1) ? (uint32_t)t : (uint32_t)(kNucBins - 1);
+}
+
+__device__ __forceinline__ uint32_t nuc_sub(float t, uint32_t b) { return nuc_bin((t - (float)b) * (float)kNucBins); }
+
+// Bin b is the coordinates from b to below nuc_end(b); the last one is open.
+__device__ __forceinline__ float nuc_end(uint32_t b)
+{
+    return b < (uint32_t)(kNucBins - 1) ? (float)(b + 1u) : INFINITY;
+}
+
+__device__ __forceinline__ void nuc_add(unsigned long long *to, unsigned long long v)
+{
+    if (v)
+        (void)__hip_atomic_fetch_add(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // This wave's rounds of the slice: round j of the wave is elements
@@ -134,13 +182,22 @@ __global__ __launch_bounds__(kThreads) void nucleus_split_kernel(SampleParams p)
 {
     __shared__ SplitLds L;
     uint32_t split, row;
-    if (nuc_place(p, split, row))
-        split_slice(p, split, row, L);
+    if (!nuc_place(p, split, row))
+        return;
+    if (split < 2 && nuc_trunc(row_topp(p, row))) {
+        unsigned long long *h = nuc_slice(p, row, split)->hist;
+#pragma unroll
+        for (int k = 0; k < kNucBins / kThreads; k++)
+            h[threadIdx.x + k * kThreads] = 0;
+    }
+    split_slice(p, split, row, L);
 }
 
 __global__ __launch_bounds__(kMergeThreads) void nucleus_weigh_kernel(SampleParams p)
 {
-    __shared__ unsigned long long hist[kNucBins];
+    // (the last bin, which may hold a quarter of a peaked row's elements, is
+    // kept kNucLast times, lane l's elements in copy l % kNucLast)
+    __shared__ unsigned long long hist[kNucBins - 1 + kNucLast];
     uint32_t split, row;
     if (!nuc_place(p, split, row))
         return;
@@ -153,9 +210,13 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_weigh_kernel(SamplePara
     float x[kNucWaveRounds][4];
     nuc_load(p, row, first, 1.0f / temp, x);
     hist[tid] = 0;
-    const float m = nuc_row_max(p, row, lane);
+    if (tid < kNucLast - 1)
+        hist[kNucBins + tid] = 0;
+    float m, z;
+    nuc_row(p, row, lane, m, z);
+    const float topp = row_topp(p, row);
     NucSlice *out = nuc_slice(p, row, split);
-    if (!nuc_trunc(row_topp(p, row))) {
+    if (!nuc_trunc(topp)) {
 #pragma unroll
         for (int j = 0; j < kNucWaveRounds; j++) {
             uint32_t s = 0;  // at most 4 x 2^24
@@ -168,22 +229,32 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_weigh_kernel(SamplePara
         }
         return;
     }
+    const float scale = nuc_scale(z, p.vocab, topp);
+    if (tid == 0 && split == 0)
+        out->scale = scale;
     __syncthreads();
+    const float lane_last = (float)(kNucBins - 1 + (lane & (kNucLast - 1)));
 #pragma unroll
     for (int j = 0; j < kNucWaveRounds; j++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const uint32_t w = nuc_weight(x[j][e] - m);
             if (w)
-                atomicAdd(&hist[nuc_bin(nuc_t(m, x[j][e]))], (unsigned long long)w);
+                atomicAdd(&hist[(uint32_t)fminf(nuc_t(m, x[j][e], scale), lane_last)], (unsigned long long)w);
         }
     __syncthreads();
-    out->hist[tid] = hist[tid];
+    uint64_t own = hist[tid];
+    if (wave == kMergeWaves - 1) {  // thread kNucBins - 1: the sum of the last bin's copies
+        const uint64_t sum = wave_inclusive_scan_u64(lane < (int)kNucLast ? hist[kNucBins - 1 + lane] : 0ull);
+        own = lane == 63 ? sum : own;
+    }
+    nuc_add(&nuc_slice(p, row, 0)->hist[tid], own);
 }
 
 __global__ __launch_bounds__(kMergeThreads) void nucleus_edge_kernel(SampleParams p)
 {
     __shared__ BlockShared bs;
+    __shared__ unsigned long long sub[kNucBins];
     uint32_t split, row;
     if (!nuc_place(p, split, row))
         return;
@@ -196,19 +267,11 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_edge_kernel(SampleParam
     const uint32_t first = split * kSplitLen + (uint32_t)wave * (256u * kNucWaveRounds) + (uint32_t)lane * 4u;
     float x[kNucWaveRounds][4];
     nuc_load(p, row, first, 1.0f / temp, x);
-    const float m = nuc_row_max(p, row, lane);
-
-    // the row's weight in bin tid, eight slices' loads in flight
-    uint64_t own = 0;
-    for (uint32_t s0 = 0; s0 < p.splits; s0 += 8) {
-        uint64_t h[8];
-#pragma unroll
-        for (uint32_t k = 0; k < 8; k++)
-            h[k] = nuc_slice(p, row, min(s0 + k, p.splits - 1))->hist[tid];
-#pragma unroll
-        for (uint32_t k = 0; k < 8; k++)
-            own += s0 + k < p.splits ? h[k] : 0ull;
-    }
+    float m, z;
+    nuc_row(p, row, lane, m, z);
+    const float scale = nuc_slice(p, row, 0)->scale;
+    const uint64_t own = nuc_slice(p, row, 0)->hist[tid];
+    sub[tid] = 0;
     uint64_t wk;
     if (tid == 0) {
         bs.cnt[0] = 0;
@@ -225,9 +288,7 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_edge_kernel(SampleParam
     const uint32_t bstar = bs.n;
 
     NucSlice *out = nuc_slice(p, row, split);
-    // t < lo: a bin above bstar's; lo <= t < hi: bin bstar. (bstar is never the
-    // last bin, which holds no weight, so hi bounds it.)
-    const float lo = (float)bstar, hi = (float)(bstar + 1u);
+    const float lo = (float)bstar, hi = nuc_end(bstar);  // t < lo: a bin above; lo <= t < hi: bin bstar
 #pragma unroll
     for (int j = 0; j < kNucWaveRounds; j++) {
         uint32_t s = 0, tot = 0;
@@ -235,10 +296,12 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_edge_kernel(SampleParam
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const uint32_t w = nuc_weight(x[j][e] - m);
-            const float t = nuc_t(m, x[j][e]);
+            const float t = nuc_t(m, x[j][e], scale);
             s += t < lo ? w : 0u;
             bal[e] = __ballot(t < hi) & ~__ballot(t < lo);
             tot += (uint32_t)__popcll(bal[e]);
+            if (bal[e] >> lane & 1)
+                atomicAdd(&sub[nuc_sub(t, bstar)], (unsigned long long)w);
         }
         if (tot) {  // one LDS atomic per wave and round
             uint32_t at = 0;
@@ -261,6 +324,7 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_edge_kernel(SampleParam
             out->rounds[wave * kNucWaveRounds + j] = sum;
     }
     __syncthreads();
+    nuc_add(&nuc_slice(p, row, 1)->hist[tid], sub[tid]);
     if (tid == 0) {
         out->members = bs.cnt[0];
         out->bstar = bstar;
@@ -271,68 +335,9 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_edge_kernel(SampleParam
 
 struct NucLds {
     unsigned long long rounds[64 * kNucRounds];
-    unsigned long long sub[kNucSubBins];
-    unsigned long long key[kNucRowMembers];  // the boundary bin: composite keys and weights
-    uint32_t w[kNucRowMembers];
-    unsigned long long skey[kSubCap];        // the boundary sub-bin
-    uint32_t sw[kSubCap];
+    unsigned long long key[kMergeThreads];  // the boundary sub-bin: composite keys and weights
+    uint32_t w[kMergeThreads];
 };
-
-// Finds, among the boundary bin's members (n of them in L.key / L.w), the one
-// at which the weight ranked (x desc, index asc) reaches thr, given `above`
-// in the bins above: tau its composite key, wp the weight up to and with it.
-// The bin is cut into kNucSubBins sub-bins (monotone again); the members of
-// the one where thr is reached are compared pairwise. False when that
-// sub-bin holds more than kSubCap (ties).
-__device__ __forceinline__ bool nuc_boundary(uint32_t n, uint32_t bstar, uint64_t above, uint64_t thr, float m,
-                                             NucLds &L, BlockShared &bs, uint64_t &tau, uint64_t &wp)
-{
-    const uint32_t tid = threadIdx.x;
-    auto sub_of = [&](uint64_t key) {
-        const float f = (nuc_t(m, rl_key_float((uint32_t)(key >> 32))) - (float)bstar) * (float)kNucSubBins;
-        return f < (float)(kNucSubBins - 1) ? (uint32_t)f : (uint32_t)(kNucSubBins - 1);
-    };
-    for (uint32_t e = tid; e < n; e += kMergeThreads)
-        atomicAdd(&L.sub[sub_of(L.key[e])], (unsigned long long)L.w[e]);
-    __syncthreads();
-    const uint64_t own = L.sub[tid];  // one sub-bin per thread
-    uint64_t total;
-    const uint64_t excl = above + block_excl_scan_u64_inl(own, total, bs);
-    if (excl < thr && excl + own >= thr) {  // exactly one thread
-        bs.res64[0] = excl;
-        bs.n = tid;
-    }
-    __syncthreads();
-    const uint64_t sub_above = bs.res64[0];
-    const uint32_t sb = bs.n;
-    for (uint32_t e0 = 0; e0 < n; e0 += kMergeThreads) {
-        const uint32_t e = e0 + tid;
-        const bool take = e < n && sub_of(L.key[e]) == sb;
-        const uint32_t pos = wave_append(take, &bs.cnt[1]);
-        if (take && pos < (uint32_t)kSubCap) {
-            L.skey[pos] = L.key[e];
-            L.sw[pos] = L.w[e];
-        }
-    }
-    __syncthreads();
-    const uint32_t ns = bs.cnt[1];
-    if (ns > (uint32_t)kSubCap)
-        return false;
-    if (tid < ns) {
-        const uint64_t ck = L.skey[tid];
-        uint64_t s = sub_above;
-        for (uint32_t j = 0; j < ns; j++)
-            s += L.skey[j] > ck ? (uint64_t)L.sw[j] : 0ull;
-        if (s < thr && s + L.sw[tid] >= thr) {  // exactly one element
-            bs.sel64 = ck;
-            bs.res64[1] = s + L.sw[tid];
-        }
-    }
-    __syncthreads();
-    tau = bs.sel64;
-    wp = bs.res64[1];
-    return true;
-}
 
 // Grid (row).
 __global__ __launch_bounds__(kMergeThreads) void nucleus_pick_kernel(SampleParams p)
@@ -361,7 +366,7 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_pick_kernel(SampleParam
     const uint32_t R = p.splits * kNucRounds;
     for (uint32_t r = tid; r < R; r += kMergeThreads)
         L.rounds[r] = nuc_slice(p, row, r / kNucRounds)->rounds[r % kNucRounds];
-    // the first 128 members of the lists this wave copies, before their
+    // the first 128 members of the lists this wave reads first, before their
     // counts are known (in bounds; past a list's count, not used)
     uint2 pv[4];
 #pragma unroll
@@ -379,43 +384,88 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_pick_kernel(SampleParam
     const float *l = p.logits + (size_t)row * p.row_stride;
 
     bool ok = m > -INFINITY && m < INFINITY;
+    float scale = 0.f;
     uint32_t bstar = kNucBins;  // every bin is in the nucleus
     uint64_t tau = 0, wp = 0;
-    uint32_t n = 0;
     if (trunc && ok) {
+        scale = head->scale;
         bstar = head->bstar;
+        const float lo = (float)bstar, hi = nuc_end(bstar);
         const uint64_t above = head->above, thr = head->thr;
-        const bool over = __ballot(cnt > (uint32_t)kNucMembers) != 0;
-        const uint32_t incl = rl_wave_incl_scan_u32(over ? 0u : cnt);
-        n = rl_readlane(incl, 63);
-        ok = !over && n <= (uint32_t)kNucRowMembers;
-        if (ok) {
-            L.sub[tid] = 0;
-            if (tid == 0)
-                bs.cnt[1] = 0;
-            // wave w copies the members of slices w, w + 8, ...
-            for (uint32_t s = wave; s < p.splits; s += kMergeWaves) {
-                const uint32_t c = rl_readlane(cnt, (int)s), at = rl_readlane(incl, (int)s) - c;
+        // ---- the sub-bin of the boundary bin where thr is reached -----------
+        if (tid == 0)
+            bs.cnt[1] = 0;
+        const uint64_t own = nuc_slice(p, row, 1)->hist[tid];
+        uint64_t total;
+        const uint64_t excl = above + block_excl_scan_u64_inl(own, total, bs);
+        if (excl < thr && excl + own >= thr) {  // exactly one thread
+            bs.res64[0] = excl;
+            bs.n = tid;
+        }
+        __syncthreads();
+        const uint64_t sub_above = bs.res64[0];
+        const uint32_t sb = bs.n;
+        // ---- the bin's members: those in the sub-bins above join their
+        // rounds, those in the sub-bin are gathered ---------------------------
+        auto member = [&](float x, uint32_t idx) {
+            const uint32_t sub = nuc_sub(nuc_t(m, x, scale), bstar);
+            const uint32_t w = nuc_weight(x - m);
+            if (sub < sb)
+                atomicAdd(&L.rounds[idx / 256u], (unsigned long long)w);
+            const bool edge = sub == sb && w != 0;
+            const uint32_t pos = wave_append(edge, &bs.cnt[1]);
+            if (edge && pos < (uint32_t)kMergeThreads) {
+                L.key[pos] = composite_key(rl_float_key(x), idx);
+                L.w[pos] = w;
+            }
+        };
+        for (uint32_t s = wave; s < p.splits; s += kMergeWaves) {  // wave w: slices w, w + 8, ...
+            const uint32_t c = rl_readlane(cnt, (int)s);
+            if (c <= (uint32_t)kNucMembers) {
                 const uint2 *src = nuc_slice(p, row, s)->list;
                 for (uint32_t i = lane; i < c; i += 64) {
                     const uint2 v = s == (uint32_t)wave && i < 128u       ? (i < 64u ? pv[0] : pv[1])
                                     : s == (uint32_t)wave + kMergeWaves && i < 128u ? (i < 64u ? pv[2] : pv[3])
                                                                           : src[i];
-                    const float xv = __uint_as_float(v.x);
-                    L.key[at + i] = composite_key(rl_float_key(xv), v.y);
-                    L.w[at + i] = nuc_weight(xv - m);
+                    member(__uint_as_float(v.x), v.y);
+                }
+            } else {
+                const uint32_t i0 = s * (uint32_t)kSplitLen + (uint32_t)lane * 4u;
+                for (uint32_t r = 0; r < (uint32_t)kNucRounds; r += kNucWaveRounds) {
+                    float x[kNucWaveRounds][4];
+                    nuc_load(p, row, i0 + 256u * r, inv_t, x);
+#pragma unroll
+                    for (int j = 0; j < kNucWaveRounds; j++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const float t = nuc_t(m, x[j][e], scale);
+                            if (t < hi && !(t < lo))
+                                member(x[j][e], i0 + 256u * (r + j) + e);
+                        }
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t ns = bs.cnt[1];
+        ok = ns <= (uint32_t)kMergeThreads;
+        if (ok) {
+            // ---- the boundary element: compared pairwise --------------------
+            if (tid < ns) {
+                const uint64_t ck = L.key[tid];
+                uint64_t s = sub_above;
+                for (uint32_t j = 0; j < ns; j++)
+                    s += L.key[j] > ck ? (uint64_t)L.w[j] : 0ull;
+                if (s < thr && s + L.w[tid] >= thr) {  // exactly one element
+                    bs.sel64 = ck;
+                    bs.res64[1] = s + L.w[tid];
                 }
             }
             __syncthreads();
-            ok = nuc_boundary(n, bstar, above, thr, m, L, bs, tau, wp);
+            tau = bs.sel64;
+            wp = bs.res64[1];
+            if (tid < ns && L.key[tid] >= tau)
+                atomicAdd(&L.rounds[(0xFFFFFFFFu - (uint32_t)L.key[tid]) / 256u], (unsigned long long)L.w[tid]);
         }
-        // the members in the nucleus join their rounds
-        if (ok)
-            for (uint32_t e = tid; e < n; e += kMergeThreads) {
-                const uint64_t ck = L.key[e];
-                if (ck >= tau)
-                    atomicAdd(&L.rounds[(0xFFFFFFFFu - (uint32_t)ck) / 256u], (unsigned long long)L.w[e]);
-            }
     }
     __syncthreads();
 
@@ -448,7 +498,7 @@ __global__ __launch_bounds__(kMergeThreads) void nucleus_pick_kernel(SampleParam
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float x = quad_at(v, e) * inv_t;
-                const uint32_t b = nuc_bin(nuc_t(m, x));
+                const uint32_t b = trunc ? nuc_bin(nuc_t(m, x, scale)) : 0u;
                 const uint64_t ck = composite_key(rl_float_key(x), i0 + e);
                 const uint32_t in = (uint32_t)(b < bstar) | ((uint32_t)(b == bstar) & (uint32_t)(ck >= tau));
                 w4[e] = nuc_weight(x - m) & (0u - in);

@@ -243,7 +243,7 @@ def test_sliced_nucleus_edges(rl, gpu, orc, olib, rows, vocab, stride):
     """Rows without top-k above the row kernel's size, over the slices: one
     slice past a boundary, rows that leave XCDs without a row, the most slices
     (64); dense and sparse boundaries, massive ties in the boundary bin (its
-    lists overflow: the exact path), -inf rows, top-p 1."""
+    sub-bin overflows: the exact path), -inf rows, top-p 1."""
     rng = np.random.default_rng(vocab + rows)
     x = np.full((rows, stride), np.float32(9.0))             # padding past vocab never read
     x[:, :vocab] = rng.standard_normal((rows, vocab), dtype=np.float32)
@@ -259,6 +259,32 @@ def test_sliced_nucleus_edges(rl, gpu, orc, olib, rows, vocab, stride):
     seeds = rng.integers(0, 2**63, rows, dtype=np.uint64)
     for p in (0.05, 0.9, 0.999, 1.0):
         _check(rl, orc, olib, x, vocab=vocab, temperature=0.9, top_k=0, top_p=p, seeds=seeds, step=int(p * 1000))
+
+
+@pytest.mark.parametrize("rows,vocab", [(11, 100003), (6, 300000)])
+def test_sliced_nucleus_spreads(rl, gpu, orc, olib, rows, vocab):
+    """Rows without top-k of every spread, over few and many slices: flat ones,
+    whose boundary bin holds thousands of members; nearly equal logits under a
+    few high ones, whose members exceed the slices' lists; peaked ones, whose
+    last bin holds much of the row; rows masked with -inf and with -1e9."""
+    stride = -(-vocab // 4) * 4
+    rng = np.random.default_rng(vocab)
+    x = np.full((rows, stride), np.float32(9.0))             # padding past vocab never read
+    x[:, :vocab] = rng.standard_normal((rows, vocab), dtype=np.float32)
+    for r, (std, spikes) in enumerate([(0.3, 0), (0.3, 5), (0.05, 5), (0.01, 1), (2.0, 0), (4.0, 0)]):
+        x[r, :vocab] *= np.float32(std)
+        x[r, rng.integers(0, vocab, spikes)] = np.float32(8.0)
+    if rows > 6:
+        x[6, :vocab][rng.random(vocab) < 0.7] = -np.inf
+        x[7, :vocab][rng.random(vocab) < 0.7] = np.float32(-1e9)
+        x[8, :vocab] *= np.float32(0.05)
+        x[8, rng.integers(0, vocab, 3)] = np.float32(7.0)
+        x[8, :vocab][rng.random(vocab) < 0.2] = -np.inf
+        x[9, : vocab // 2] -= np.float32(3.0)                # the members in half of the slices
+        x[10, :vocab] = np.float32(2.0) + np.float32(1e-3) * x[10, :vocab]
+    seeds = rng.integers(0, 2**63, rows, dtype=np.uint64)
+    for p in (0.1, 0.7, 0.95, 0.999999):
+        _check(rl, orc, olib, x, vocab=vocab, temperature=1.0, top_k=0, top_p=p, seeds=seeds, step=int(p * 1000))
 
 
 def test_sliced_nucleus_per_row_parameters(rl, gpu, orc, olib):
