@@ -1123,23 +1123,52 @@ AppendParams append_or_none(const rl_kv_append_args_t *append)
 namespace {
 
 // Fused-kernel shapes whose step is faster as the decode step and then the
-// sampling, each in its own kernels:
-//  - rows without top-k above 32,768 logits, which a sampling workgroup would
-//    stream twice from one compute unit and rl_hip_sample spreads over slices
-//    (64 rollouts of U[512, 4,096], 128,256 logits, top-p: 163 us against 179;
-//    200 of U[100, 1,000], 60,000 logits: 141 against 252);
-//  - batches of few rows (rl_attn_few_rows) with rows of 16,384 logits and
-//    more, bound by latency (4 x U[100, 1,000] with 32,000 logits, top-k 50:
-//    23.8 us against 26.9; 2 x U[1,000, 8,000], 128,256 logits: 33.2 against
-//    53.5; but 1 x U[100, 300] with 4,000 logits 13.8 against 12.7).
+// sampling, each in its own kernels (us, GQA 4, d128, two calls against fused):
+//  - batches of few rows (rl_attn_few_rows), bound by latency, with
+//    - more than 32,768 logits (2 x U[1,000, 8,000], 128,256 logits, top-k 50:
+//      34.0 against 52.1; 1 x 1,024, top-p: 31 against 116);
+//    - 16,384 and more, greedy or with top-k, when the attention is longer
+//      than 512 tokens (4 x U[1,000, 2,000], 32,000 logits, top-k 50: 26.5
+//      against 32.9; 8 x U[350, 700] 25.5 against 28.7; but 8 x U[50, 100]
+//      23.4 against 21.5, and 1 x U[100, 300] with 4,000 logits 13.8 against
+//      12.7);
+//    - 16,384 and more without top-k, which the fused kernel streams twice (2 x
+//      U[200, 400], top-p 1: 18.6 against 26.1 at 16,384 logits; top-p 0.9:
+//      32.8 against 34.2 at 20,000, 24.7 against 41.5 at 32,000, but 35.1
+//      against 31.3 at 17,000: rl_hip_sample's row kernel wants full registers);
+//  - larger batches with rows without top-k above 32,768 logits, whose chain of
+//    rows on one sampling workgroup (0.9 ns a logit) is long beside the
+//    attention it should hide under: rl_hip_sample spreads it over slices. The
+//    host knows only max_ctx, so the attention is taken at 5.5 TB/s over that
+//    many tokens a rollout; the line lies where contexts of half to all of
+//    max_ctx break even, at 0.55 of it for one row per workgroup (64 x
+//    U[512, 4,096], 128,256 logits: 160 against 179; 64 x U[750, 1,500]: 65,536
+//    logits 97 against 102, 40,000 logits 95 against 86; 32 x U[2,048, 4,096],
+//    40,000: 107 against 98; 64 x 16,384, 128,256: 758 against 755) and at 0.35
+//    for more (128 x U[2,048, 4,096], 128,256: 354 against 375, 65,536: 329
+//    against 322; 256 x U[750, 1,500], 40,000: 282 against 303; 200 x U[100,
+//    1,000], 60,000: 137 against 251).
 // The caller's workspace decides whether they can: one sized for other
 // sampling arguments keeps the fused kernel. So does the ring-driven step,
 // whose launched and self-scheduled forms sample with the same code.
 bool one_after_the_other(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp)
 {
-    const bool no_topk = !samp->top_k && (samp->top_k_all == 0 || samp->top_k_all >= samp->vocab);
-    return (no_topk && !samp->greedy && samp->vocab > RL_ROW_SAMPLER_VOCAB) ||
-           (samp->vocab >= 16384 && rl_attn_few_rows(attn));
+    const bool whole =
+        !samp->greedy && !samp->top_k && (samp->top_k_all == 0 || samp->top_k_all >= samp->vocab);
+    const bool nucleus = samp->top_p || (samp->top_p_all > 0.f && samp->top_p_all < 1.f);
+    if (rl_attn_few_rows(attn)) {
+        if (samp->vocab > RL_ROW_SAMPLER_VOCAB)
+            return true;
+        return whole ? samp->vocab >= (nucleus ? 20000u : 16384u) : samp->vocab >= 16384 && attn->max_ctx > 512;
+    }
+    if (!whole || samp->vocab <= RL_ROW_SAMPLER_VOCAB)
+        return false;
+    const uint32_t wgs = split_in_of(attn, samp).sample_wgs;
+    const uint32_t rows = (samp->rows + wgs - 1) / wgs;  // one after another on a sampling workgroup
+    const double chain_ns = 0.9 * rows * samp->vocab;
+    const double attn_ns =
+        (double)attn->batch * attn->kv_heads * attn->max_ctx * attn->layout.head_dim * 4.0 / 5500.0;
+    return chain_ns >= (rows > 1 ? 0.35 : 0.55) * attn_ns;
 }
 
 size_t apart_ws(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp)

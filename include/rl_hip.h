@@ -131,7 +131,12 @@ int rl_hip_attn_decode(const rl_attn_decode_args_t *args);
  * query_prepare_kernel, cu/query_producer.cu:5-26). logits[r][v] =
  * sum_k x[r][k] * w[v][k]: bf16 operands (w stored like an lm_head weight,
  * one row of `hidden` per vocabulary entry), fp32 accumulate and output, on
- * MFMA. `hidden` must be a multiple of 64; x and w strides multiples of 8. */
+ * MFMA. `hidden` must be a multiple of 64; x and w strides multiples of 8.
+ * A call's results are the same at every repetition. The order of the fp32
+ * sums over `hidden` depends on the number of rows (up to 32, 64, 128 and
+ * above) and, up to 128 rows, on the block of vocabulary entries: the same row
+ * of x in a call of another size, or two equal rows of w, can differ in the
+ * last bits. */
 typedef struct {
     const void *x;               /* device [rows][x_stride] bf16 */
     const void *w;               /* device [vocab][w_stride] bf16 */
@@ -598,20 +603,25 @@ int rl_hip_decode_step(const rl_attn_decode_args_t *attn, const rl_kv_append_arg
  * step produced: rl_hip_decode_step(attn, append) and rl_hip_sample(samp) in
  * one persistent launch that streams both from HBM side by side, plus the
  * attention merge with the append. samp must not read what attn writes (its
- * logits are the other micro-batch's). Tokens, logprobs and the appended
- * KV equal the two calls'; the attention is the same fp32 online-softmax
- * math with the rows split at other tile positions (fixed for a given set
- * of contexts, so repeated calls give the same bits), within 1e-4 of fp64
+ * logits are the other micro-batch's). Tokens and the appended KV equal the
+ * two calls', and so do the logprobs up to the order in which their
+ * log-sum-exp is added up in fp32 (within 2e-5); the attention is the same
+ * fp32 online-softmax math with the rows split at other tile positions (fixed
+ * for a given set of contexts, so repeated calls give the same bits), within
+ * 1e-4 of fp64
  * like rl_hip_attn_decode. The workspace (size from
  * rl_hip_decode_sample_step_workspace) holds the step's tile prefix and
  * partials; it needs no initialisation. append may be NULL: the attention
  * and the sampling without a KV append. Shapes whose tiles do not fit the
  * fused kernel's LDS (GQA groups of 8 at head_dim 128, batches above 1,024)
  * run rl_hip_decode_step (rl_hip_attn_decode without an append) and then
- * rl_hip_sample on the same workspace, with exactly their results; so do, as
- * long as the workspace was sized for them, samplings without top-k of more
- * than 32,768 logits and batches of few rows with 16,384 logits or more,
- * which are faster that way. */
+ * rl_hip_sample on the same workspace, with exactly their results. So do, with
+ * a workspace sized for the same arguments, the calls that are faster that
+ * way: batches of few rows with 16,384 logits or more, and samplings without
+ * top-k of more than 32,768 logits beside an attention that is short next to
+ * them. A smaller workspace, as other sampling arguments need, keeps such a
+ * call on the fused kernel: the same tokens and KV, the logprobs and the
+ * attention within the bounds above. */
 size_t rl_hip_decode_sample_step_workspace(const rl_attn_decode_args_t *attn, const rl_sample_args_t *samp);
 int rl_hip_decode_sample_step(const rl_attn_decode_args_t *attn, const rl_kv_append_args_t *append,
                               const rl_sample_args_t *samp, void *workspace, size_t workspace_bytes);
@@ -624,10 +634,12 @@ int rl_hip_decode_sample_step(const rl_attn_decode_args_t *attn, const rl_kv_app
  * that step was given as its workspace). So the rows of attn are complete
  * only after the next step (or rl_hip_decode_pipeline_flush) has run; rows
  * that one piece covered are written at once. Tokens and the appended KV
- * equal rl_hip_decode_sample_step's, and so do the logprobs (to fp32 rounding
- * where that call runs its two steps apart); the attention is its fp32 math
- * (bit for bit when the split is the same, as at the first step: the merge
- * work of the sampling waves shifts the split otherwise), within 1e-4 of fp64. prev_attn NULL: nothing to merge (the first step). The two micro-batches alternate, each with its own
+ * equal rl_hip_decode_sample_step's, and the logprobs too, bit for bit where
+ * that call takes its fused kernel and within 2e-5 where it runs its two steps
+ * apart; the attention is its fp32 math (bit for bit when the split is the
+ * same, as at the first step: the merge work of the sampling waves shifts the
+ * split otherwise), within 1e-4 of fp64. prev_attn NULL: nothing to merge (the
+ * first step). The two micro-batches alternate, each with its own
  * workspace of rl_hip_decode_sample_step_workspace bytes; prev_attn must
  * have attn's heads, dtype and layout, and prev_append must not write what
  * attn reads (the other micro-batch's blocks; a slot at or past a row's

@@ -613,11 +613,18 @@ def test_step_append_wave(rl, gpu, orc, olib, batch, heads):
     (40, 900, 40, 40000, dict(temperature=0.9, top_k=0, top_p=0.9, seed=4, step=2)),
     (70, 300, 9, 32772, dict(temperature=1.0, top_k=0, top_p=1.0, seed=5, step=3)),
     (3, 700, 3, 16384, dict(temperature=0.8, top_k=50, top_p=0.9, seed=6, step=4)),
-    (1, 5000, 17, 32000, dict(temperature=1.0, top_k=0, top_p=0.9, seed=7, step=5))])
+    (1, 5000, 17, 32000, dict(temperature=1.0, top_k=0, top_p=0.9, seed=7, step=5)),
+    # the other side of each line: the fused kernel
+    (40, 3000, 40, 32772, dict(temperature=0.9, top_k=0, top_p=0.9, seed=8, step=6)),
+    (3, 512, 3, 16384, dict(temperature=0.8, top_k=50, top_p=0.9, seed=9, step=7)),
+    (2, 700, 2, 19996, dict(temperature=1.0, top_k=0, top_p=0.9, seed=10, step=8))])
 def test_steps_one_after_the_other(rl, gpu, orc, olib, batch, hi, rows, vocab, samp):
     """Fused-kernel shapes that run as the decode step and then the sampling
-    (long rows without top-k, few rows): against the oracle, and on a
-    workspace of the fused kernel's own size, which keeps that kernel."""
+    (long rows without top-k beside a short attention, few rows), and shapes
+    just outside them: against the oracle, and on a workspace of the fused
+    kernel's own size, which keeps that kernel. Logprobs of the two ways and of
+    the pipelined step within 2e-5: two fp32 sums, each term at most 100
+    roundings deep (12 x 10^-6 together), and the roundings of a logprob."""
     rng = np.random.default_rng(vocab + batch)
     w = synth.make_decode(61, batch, 32, 8, 128, 1, hi, max_ctx=hi)
     kn, vn = _kv_rows(rng, w)
@@ -642,11 +649,13 @@ def test_steps_one_after_the_other(rl, gpu, orc, olib, batch, hi, rows, vocab, s
     rl.decode_sample_step(a, None, s, ws)
     rl.sync()
     assert np.array_equal(tok.download(np.uint32, rows), want)
+    assert np.abs(lp.download(np.float32, rows) - res[0][4]).max() < 2e-5
     o32 = out32.download(np.float32, (batch, 32, 128))
     assert (gh.rownorm_err(o32, orc.attn_f64(olib, w, 0)) < 1e-4).all()
     tok.upload(np.zeros(rows, np.uint32))     # the pipelined form needs no more than that workspace either
     rl.decode_pipeline_step(a, s, ws)
     rl.sync()
     assert np.array_equal(tok.download(np.uint32, rows), want)
+    assert np.abs(lp.download(np.float32, rows) - res[0][4]).max() < 2e-5
     for b in list(bufs.values()) + [out, out32, tok, lp, ws]:
         b.close()
