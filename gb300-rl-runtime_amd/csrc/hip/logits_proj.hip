@@ -6,14 +6,14 @@
 // like an lm_head weight, one row of K per vocabulary entry, so both
 // operands are K-contiguous.
 //
-//  tiles   one 512-thread workgroup (8 waves, 4 along M x 2 along N) per
-//          output tile, K in steps of 64:
-//          - up to 128 rows: tiles of 32, 64 or 128 rows by 64 or 128
-//            (logits_proj_rows_kernel, below).
-//          - up to 256 rows: 256 x 128 tiles, waves of 64 x 64 (4 x 4 MFMA
-//            blocks of 16 x 16), a 3-stage LDS ring (144 KiB). Every W tile
-//            is read by exactly one workgroup, and the grid (one workgroup
-//            per 128 vocabulary rows) fits the device in one round.
+//  tiles   one workgroup per output tile, K in steps of 64:
+//          - up to 128 rows: tiles of 32, 64 or 128 rows by 64 or 128 of 4 or
+//            8 waves (logits_proj_rows_kernel, below).
+//          - 129 to 256 rows: 256 x 128 tiles of 512 threads (8 waves, 4 along
+//            M x 2 along N), waves of 64 x 64 (4 x 4 MFMA blocks of 16 x 16),
+//            a 3-stage LDS ring (144 KiB). Every W tile is read by exactly one
+//            workgroup, and the grid (one workgroup per 128 vocabulary rows)
+//            fits the device in one round.
 //          - above 256 rows: 256 x 256 tiles, waves of 64 x 128, a 2-stage
 //            ring (128 KiB). The larger wave tile reads fewer LDS bytes per
 //            MFMA, and at 512 rows the grid is again one round.
@@ -209,12 +209,18 @@ __global__ __launch_bounds__(kThreads) void logits_proj_kernel(ProjParams p)
 // on X rows that are not there, and its one 144 KiB workgroup per compute unit
 // keeps 32 KiB of W in flight. Here every workgroup covers all rows of X, so W
 // is read once, and the tiles are small: WN waves of TNR x 16 vocabulary rows
-// each, a 3-stage ring of 12 to 32 KiB stages, so that up to four workgroups
-// share a compute unit and fill each other's barrier waits. (Deeper rings with
-// fewer workgroups were slower: 6 stages 52 us against 45 at 24 rows.)
+// each, a 3-stage ring of 12, 24 or 32 KiB stages, so that up to 32 and 64
+// rows four and two workgroups share a compute unit and fill each other's
+// barrier waits (at 128 rows one, of 96 KiB). (Deeper rings with fewer
+// workgroups were slower: 6 stages 52 us against 45 at 24 rows.)
 // Each workgroup starts at another K step and wraps, so that the workgroups
 // that run at once read W at different columns; all starting at 0 they read
-// column k of rows 8 KiB apart together (24 rows 51.8 us against 45.5).
+// column k of rows 8 KiB apart together (32,000 x 4,096 at 24 rows 56.5 us
+// against 46.2, at 64 rows 66.0 against 48.0, at 128 rows 58.8 against 56.4;
+// a pitch that is no power of two does not care, 27,173 x 1,408 12.5 both
+// ways). The price: the order of a logit's sum depends on its block, so equal
+// rows of W can differ in the last bits (rl_hip.h says so). Delaying the
+// workgroups against each other instead (s_sleep) did not help: 56.1 us.
 // Measured back to back over three copies of W, 32,000 x 4,096 (us, against
 // the 256 x 128 tile): 1 row 44.4 (60.4), 24 rows 45.5 (62.9), 64 rows 48.8
 // (65.4), 128 rows 55.9 (70.5); 20 rows of 17,393 x 2,048 12.3 (30); 1 row of

@@ -62,6 +62,36 @@ def test_projection_few_rows(rl, gpu, rows, vocab, hidden):
     _case(rl, rows, vocab, hidden, seed=rows + vocab + hidden)
 
 
+def test_projection_sum_order(rl, gpu):
+    """What a caller may rely on: a repeated call gives the same bits; the same
+    row of x in calls of other sizes, and equal rows of w in other blocks of
+    the vocabulary, agree within the bound of two fp32 sums in any order."""
+    rng = np.random.default_rng(91)
+    vocab, hidden = 1000, 512
+    x = synth.f32_to_bf16(rng.standard_normal((257, hidden), dtype=np.float32))
+    w = synth.f32_to_bf16(rng.standard_normal((vocab, hidden), dtype=np.float32) * np.float32(0.02))
+    w[700:720] = w[10:30]
+    mag = np.abs(synth.bf16_to_f32(x[:1]).astype(np.float64)) @ np.abs(synth.bf16_to_f32(w).astype(np.float64)).T
+    bound = 2.0 * (hidden - 1) * 2.0**-24 * mag[0]
+    dw, first = rl.DeviceBuffer.from_array(w), []
+    for rows in (1, 32, 33, 64, 65, 128, 129, 257):
+        print(f"[proj] rows={rows} vocab={vocab} hidden={hidden}, twice", flush=True)
+        dx, out = rl.DeviceBuffer.from_array(x[:rows]), rl.DeviceBuffer(rows * vocab * 4)
+        got = []
+        for _ in range(2):
+            rl.logits_proj(dx, dw, out, rows, vocab, hidden)
+            rl.sync()
+            got.append(out.download(np.float32, (rows, vocab)))
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+        first.append(got[0][0].astype(np.float64))
+        dx.close()
+        out.close()
+    for l in first:
+        assert np.all(np.abs(l - first[0]) <= bound)
+        assert np.all(np.abs(l[700:720] - l[10:30]) <= bound[10:30])
+    dw.close()
+
+
 def test_projection_loop_shape(rl, gpu):
     """256 x 4096 -> 32,000 (the rollout loop's 256 slots, the tile whose
     waves split the X and W copies): every column of 24 rows, every row of
