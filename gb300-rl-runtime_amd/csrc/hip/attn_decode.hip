@@ -252,7 +252,7 @@ __global__ __launch_bounds__(THREADS) void attn_merge_kernel(AttnParams p, Appen
 // workgroups' compute units only, hence the rule at rows_split.
 // Measured, calls back to back (us, against attn_decode_kernel +
 // attn_merge_kernel; GQA 4, d128, bf16, with the append): 1 x 128 tokens
-// (without) 5.4 (10.2), 1 x 517 8.8 (12.9), 1 x 4,096 12.9 (31.9), 4 x
+// (without) 5.4 (10.2), 1 x 517 8.2 (12.9), 1 x 4,096 12.9 (31.9), 4 x
 // U[100, 1,024] 9.5 (15.4), 8 x U[512, 4,096] 23.2 (25.8), 32 x U[100, 200]
 // 10.8 (15.4); d64: 2 x U[64, 2,048] 9.2 (18.8).
 template <int D>

@@ -7,7 +7,7 @@
 // are 19 MB, 4 us of HBM. Here every pass over the row is a launch over
 // (slice, row) workgroups, and only the last, which touches about a thousand
 // elements, is one workgroup per row. Passes after the first read the logits
-// from L2 / Infinity Cache. Every sum is of integers, so the token does not
+// from the Infinity Cache. Every sum is of integers, so the token does not
 // depend on the split.
 //
 //  nucleus_split_kernel    slice maxima and exp sums (split_slice of
@@ -83,11 +83,10 @@ __device__ __forceinline__ NucSlice *nuc_slice(const SampleParams &p, uint32_t r
     return reinterpret_cast<NucSlice *>(p.cand + ((size_t)row * p.splits + split) * kCandStride);
 }
 
-// The (slice, row) of a workgroup. Workgroup b runs on XCD b % 8, each XCD
-// with its own L2: a row's slices all go to XCD row % 8, in every pass and in
-// the pick, so that the histograms and lists one pass leaves for the next,
-// and (up to about 64 rows of 128,256) the logits, are read from the L2 that
-// wrote them. False for a workgroup past the last row.
+// The (slice, row) of a workgroup. Workgroup b runs on XCD b % 8: a row's
+// slices all go to XCD row % 8, in every pass and in the pick. (Each pass
+// still fetches its 19 MB of logits at 37 rows from beyond the L2s.) False for
+// a workgroup past the last row.
 __device__ __forceinline__ bool nuc_place(const SampleParams &p, uint32_t &split, uint32_t &row)
 {
     const uint32_t local = blockIdx.x / kNucXcds;
