@@ -245,8 +245,8 @@ __global__ __launch_bounds__(THREADS) void attn_merge_kernel(AttnParams p, Appen
 // merge that first finds its partials, up to 256 per row. Here the grid names
 // the row: RW waves of a workgroup stream contiguous shares of its tiles,
 // both stages' copies fly (CtxRow), and the waves' partials are merged in the
-// stage buffers they no longer need. A row has one workgroup, and the step one launch, or up to
-// kRowsMaxSplit with one partial each for rows_merge_kernel.
+// stage buffers they no longer need. A row has one workgroup, or up to
+// kRowsMaxSplit with one partial each for rows_merge_kernel, which appends too.
 // Bound: latency, about 1 us per tile and wave (copy, then a chain of MFMAs
 // and cross-lane steps) and 2 us per launch; a row's KV comes through its
 // workgroups' compute units only, hence the rule at rows_split.
@@ -261,98 +261,15 @@ constexpr int rows_waves_of()
     return D == 64 ? 16 : 8;
 }
 
-// Workgroups of a launch that are done with every KV read, counted in eight
-// groups of their own cache line and one counter above (an atomic on one
-// address takes about 30 ns, so 256 workgroups on one would queue). The last
-// workgroup of a group clears its counter and counts the group; the last
-// group's clears the top one. One set per device serves every caller because
-// only launches that follow one another use it: those made directly on the
-// library's one stream. A step recorded into a graph, which may be replayed
-// on any stream beside others, appends in a second launch (launch_rows), as
-// every other route of a step does. So each launch finds zeros.
-constexpr uint32_t kDoneGroups = 8;
-constexpr uint32_t kDoneStride = 32;  // counters 128 bytes apart
-__device__ uint32_t g_rows_done[(kDoneGroups + 1) * kDoneStride];
-
-__device__ __forceinline__ bool last_workgroup(uint32_t wg, uint32_t wgs)
-{
-    const uint32_t groups = wgs <= 2 * kDoneGroups ? 1u : kDoneGroups;  // (few workgroups: one counter)
-    const uint32_t grp = wg % groups, in_grp = (wgs - grp + groups - 1) / groups;
-    uint32_t *c = g_rows_done + grp * kDoneStride, *top = g_rows_done + kDoneGroups * kDoneStride;
-    if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != in_grp - 1)
-        return false;
-    __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (groups == 1)
-        return true;
-    if (__hip_atomic_fetch_add(top, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != groups - 1)
-        return false;
-    __hip_atomic_store(top, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
-}
-
-// The append of the whole batch by one workgroup. The step's contract is that
-// every context is read before any token is appended (a row may read a block
-// another row appends to), so the launch's last workgroup to finish its reads
-// appends for all. Writing after reads needs no cache maintenance: the reads
-// were complete before their workgroup counted itself.
-constexpr uint32_t kRowsAppendMax = 64;  // (rollout, kv head) rows one workgroup appends
-
-// Thread tid's 16-byte chunks of the batch's append (chunk tid + k nthr of
-// all rows' K and V, rows in (b, g) order): loaded and addressed before the
-// attention starts, stored by store() after it. Without a copy-on-write
-// source (those rows take append_row, one wave each).
-template <int N>
-struct AppendChunks {
-    uint8_t *dst[N];  // NULL: nothing to write
-    rl_u32x4 v[N];
-
-    __device__ __forceinline__ void load(const AppendParams &p, uint32_t rows, uint32_t tid, uint32_t nthr)
-    {
-        // (each loop's loads go out together)
-        const uint32_t chunks = p.row_bytes / 16, items = rows * 2 * chunks;
-        uint32_t at[N], b[N], trow[N], pos[N], blk[N];
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-            const uint32_t i = min(tid + k * nthr, items - 1);
-            const uint32_t r = i / (2 * chunks), plane = i / chunks % 2, c = i % chunks;
-            at[k] = plane * (p.token_count * p.row_bytes) + c * 16;
-            b[k] = r / p.kv_heads;
-            trow[k] = r;
-            pos[k] = p.positions[b[k]];
-            v[k] = *(const rl_u32x4 *)((plane ? p.v_new : p.k_new) + (size_t)r * p.row_bytes + c * 16);
-        }
-        // a position past the table (a row that appends nothing) reads neither
-        // the row map nor the table
-        bool ok[N];
-#pragma unroll
-        for (int k = 0; k < N; k++)
-            ok[k] = tid + k * nthr < items && pos[k] / p.token_count < p.table_stride;
-        if (p.row_map) {
-#pragma unroll
-            for (int k = 0; k < N; k++)
-                if (ok[k])
-                    trow[k] += (p.row_map[b[k]] - b[k]) * p.kv_heads;
-        }
-#pragma unroll
-        for (int k = 0; k < N; k++)
-            blk[k] = ok[k] ? p.table[(size_t)trow[k] * p.table_stride + pos[k] / p.token_count] : 0u;
-#pragma unroll
-        for (int k = 0; k < N; k++)
-            dst[k] = ok[k] && blk[k] < p.arena_blocks
-                         ? p.arena + (uint64_t)blk[k] * p.block_bytes + at[k] + pos[k] % p.token_count * p.row_bytes
-                         : nullptr;
-    }
-
-    __device__ __forceinline__ void store() const
-    {
-#pragma unroll
-        for (int k = 0; k < N; k++)
-            if (dst[k])
-                *(rl_u32x4 *)dst[k] = v[k];
-    }
-};
-
-// The append on its own, after the rows of a larger batch.
+// The append on its own, after the rows whose launch needs no merge. (The
+// launch's workgroups cannot append by themselves: every context is read
+// before any token is written, also a block that another row appends to. A
+// count of the workgroups that are done, with the last one appending for all,
+// would need counters that start at zero and belong to the call; one set for
+// every caller is not safe beside steps on other streams. It was faster only
+// at one and two rollouts, 6.7 to 8.9 us against 7.5 to 9.5 up to 250 tokens;
+// from four on it was slower, 8 x U[125, 250] 9.8 us against 8.7, and so was
+// the attention alone, 6.9 against 6.6.)
 __global__ __launch_bounds__(64) void rows_append_kernel(AppendParams p)
 {
     append_row(p, blockIdx.y, blockIdx.x, threadIdx.x, 64);
@@ -425,7 +342,7 @@ __device__ __forceinline__ uint32_t wave_share(uint32_t w, uint32_t nu, uint32_t
 }
 
 template <int D, int G, int DT, int TPB>
-__global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(AttnParams p, AppendParams ap)
+__global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(AttnParams p)
 {
     using C = Cfg<D, G, DT, TPB>;
     constexpr int RW = rows_waves_of<D>();
@@ -441,11 +358,6 @@ __global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(Attn
     const uint32_t row = wg / S, s = wg % S;
     const uint32_t b = row / p.kv_heads, g = row % p.kv_heads;
     const uint32_t cin = rl_sload(p.ctx + b);
-    constexpr int NCH = (int)(kRowsAppendMax * 2 * C::RB / 16 / (RW * 64));
-    AppendChunks<NCH> app;
-    const bool whole = ap.arena && !ap.cow_src;
-    if (whole)
-        app.load(ap, gridDim.x, threadIdx.x, RW * 64);
     const bool bad = cin > p.max_ctx;
     const uint32_t nu = tiles_of(p, cin);
     const uint32_t nw = min(RW * S, nu);  // waves of the row with tiles, ...
@@ -505,20 +417,6 @@ __global__ __launch_bounds__(rows_waves_of<D>() * 64) void attn_rows_kernel(Attn
             if (p.out_f32)
                 p.out_f32[obase + e] = v;
         }
-    }
-    if (!ap.arena)
-        return;
-    uint32_t *last = (uint32_t *)lds_q;  // (the q slots are free)
-    if (threadIdx.x == 0)
-        *last = last_workgroup(wg, gridDim.x);
-    __syncthreads();
-    if (!*last)
-        return;
-    if (whole) {
-        app.store();
-    } else {
-        for (uint32_t r = wave; r < gridDim.x; r += RW)
-            append_row(ap, r / ap.kv_heads, r % ap.kv_heads, lane, 64);
     }
 }
 }  // namespace
@@ -604,21 +502,9 @@ template <int D, int G, int DT, int TPB>
 int launch_rows(AttnParams p, const AppendParams &ap, uint32_t split)
 {
     const uint32_t rows = p.batch * p.kv_heads;
-    // The append in the launch itself: for steps whose launches are ordered by
-    // the library stream (g_rows_done); not while it is captured.
-    AppendParams in = ap;
-    if (split > 1 || rows > kRowsAppendMax) {
-        in.arena = nullptr;
-    } else if (ap.arena) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (rl_check_hip(hipStreamIsCapturing(rl_stream(), &st), "hipStreamIsCapturing"))
-            return -1;
-        if (st != hipStreamCaptureStatusNone)
-            in.arena = nullptr;
-    }
     p.nwaves = split;
     hipLaunchKernelGGL((attn_rows_kernel<D, G, DT, TPB>), dim3(rows * split), dim3(rows_waves_of<D>() * 64), 0,
-                       rl_stream(), p, in);
+                       rl_stream(), p);
     if (rl_check_launch("attn_rows_kernel launch"))
         return -1;
     if (split > 1) {
@@ -630,7 +516,7 @@ int launch_rows(AttnParams p, const AppendParams &ap, uint32_t split)
             hipLaunchKernelGGL((rows_merge_kernel<D, G, DT, kRowsMaxSplit>), grid, dim3(threads), 0, rl_stream(), p, ap);
         return rl_check_launch("rows_merge_kernel launch");
     }
-    if (ap.arena == in.arena)
+    if (!ap.arena)
         return 0;
     hipLaunchKernelGGL(rows_append_kernel, dim3(p.kv_heads, p.batch), dim3(64), 0, rl_stream(), ap);
     return rl_check_launch("rows_append_kernel launch");
@@ -938,11 +824,6 @@ int rl_attn_scratch_setup(int device)
                      kScratchDevices);
         return -1;
     }
-    // (no launch of an earlier session is left: rl_hip_close waits)
-    void *done = nullptr;
-    if (rl_check_hip(hipGetSymbolAddress(&done, HIP_SYMBOL(g_rows_done)), "hipGetSymbolAddress(g_rows_done)") ||
-        rl_check_hip(hipMemset(done, 0, sizeof(g_rows_done)), "hipMemset(g_rows_done)"))
-        return -1;
     if (g_scratch_dev[device])
         return 0;
     void *p = nullptr;

@@ -91,8 +91,8 @@ def test_decode_step_equals_attention_then_append(rl, gpu, orc, olib, dtype):
     gh.check_attn(o16b.reshape(B, QH, D), o32b, orc.attn_f64(olib, w, 0 if dtype == "bf16" else 1), dtype)
 
 
-# the kernels for few rows: one workgroup per row with the append in the
-# launch (up to 64 rows) or after it, up to 8 and more workgroups per row
+# the kernels for few rows: one workgroup per row with the append after it, up
+# to 8 and more workgroups per row with the append beside their merge
 @pytest.mark.parametrize("batch,qh,kvh,d,tpb,dtype,hi", [
     (1, 32, 8, 128, 16, "bf16", 256), (3, 16, 8, 128, 16, "fp16", 200), (30, 8, 8, 64, 32, "bf16", 500),
     (5, 32, 8, 64, 16, "fp16", 3000), (8, 64, 8, 128, 32, "bf16", 1500), (1, 8, 1, 128, 16, "bf16", 7000),

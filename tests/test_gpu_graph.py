@@ -68,10 +68,10 @@ def test_captured_decode_step_replays_exactly(rl, gpu):
 
 
 def test_captured_few_row_steps_on_two_streams(rl, gpu):
-    """Two recorded decode steps of few rows (whose direct form counts its
-    workgroups in memory of the library) replayed side by side on two streams
-    of the caller: each replay gives the bytes of the direct call, the
-    appended token included."""
+    """Two recorded decode steps of few rows, with workspaces and arenas of their
+    own, replayed side by side on two streams of the caller: each replay gives
+    the bytes of the direct call, the appended token included (no state of the
+    library is shared between them)."""
     hip = rl.lib()  # (its own HIP runtime: symbols of a dependency)
     B, QH, KVH, D, TPB = 4, 32, 8, 128, 16
     steps, streams = [], []
